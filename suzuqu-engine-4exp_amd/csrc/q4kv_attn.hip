@@ -3624,6 +3624,16 @@ static bool held_matches(const AttnArgs &a) {
 template <int KIND, int MODE>
 static bool launch_kind(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t gqa,
                         const OutProj *op = nullptr, PartBuf pb = lib_part()) {
+    if constexpr (MODE == MODE_DENSE && KIND != Q4KV_F32) {
+        /* many tokens over one cache: the dense prefill kernel */
+        const uint32_t n_tok = n_items / a.n_kvh;
+        const bool al = ((((uintptr_t)a.kc) | ((uintptr_t)a.vc)) & 15u) == 0u;
+        if (q4kv_dense_takes(KIND, a.hd, n_tok, a.n_kvh, gqa, max_n, al)) {
+            if (!q4kv_flush()) return false;
+            return q4kv_dense_launch(KIND, a.hd, a.q, a.kc, a.vc, a.gate, a.out, pb.ptr, pb.cap,
+                                     a.n_head, a.n_kvh, n_tok, a.kv_base, a.max_kv, a.scale_log2);
+        }
+    }
     if (any_shape(a.hd, gqa)) {
         if (!q4kv_flush()) return false;
         if constexpr (IS_STEP(MODE)) {

@@ -46,6 +46,15 @@ bool q4kv_flush(void);
 extern "C" bool q4kv_scratch_init(void);
 
 
+/* Dense causal attention of many tokens (q4kv_dense.hip): whether it takes
+ * a call, and its launches; part holds the partials of split tiles. */
+bool q4kv_dense_takes(int kind, uint32_t hd, uint32_t n_tok, uint32_t n_kvh, uint32_t gqa,
+                      uint32_t max_n, bool rows16);
+bool q4kv_dense_launch(int kind, uint32_t hd, const float *q, const void *kc, const void *vc,
+                       const float *gate, float *out, float *part, size_t cap, uint32_t n_head,
+                       uint32_t n_kvh, uint32_t n_tok, uint32_t kv_base, uint32_t max_kv,
+                       float scale_log2);
+
 /* The append half of q4_hip_qsa_step_batch for widths the fused kernel
  * does not cover: d_step_descs is a device array of q4kv_step_desc. */
 bool q4kv_append_steps(const void *d_step_descs, uint32_t n_desc, uint32_t n, uint32_t bpt,

@@ -1,0 +1,98 @@
+"""The dense prefill kernel (q4kv_dense.hip: many tokens, 64 / 128 / 256 dims,
+q8_0 and f16 caches) against the oracle where it can go wrong: column tiles
+of 128 (tokens x query heads) with remainders, passes of 32 to 128 positions,
+tiles split over workgroups and merged, a cache that ends before the tokens
+do, unaligned queries, and values that are not finite in rows that only some
+tokens see."""
+import numpy as np
+import pytest
+
+import q4kv
+from gpu_util import note, quantize_on_gpu
+from synth import assert_attn_close, heads
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(rt, q, gate, kc, vc, kind, n_kvh, base, max_kv, shift=0):
+    """One decode_n call; shift moves q, gate and out by that many floats."""
+    n_tok, n_head, hd = q.shape
+    bufs = [rt.alloc(q.nbytes + 16) for _ in range(3)]
+    for b, x in zip(bufs, (q, gate)):
+        rt.h2d(b + 4 * shift, x)
+    dq, dg, do = (b + 4 * shift for b in bufs)
+    assert rt.lib.q4_hip_qsa_decode_n(dq, kc, vc, dg, do, n_head, n_kvh, hd, n_tok, base, max_kv,
+                                      1.0 / np.sqrt(hd), kind)
+    rt.sync()
+    got = rt.download(do, q.nbytes, np.float32).reshape(q.shape)
+    for b in bufs:
+        rt.free(b)
+    return got
+
+
+def _inputs(seed, kind, n_head, n_kvh, hd, n_tok, ctx):
+    rng = np.random.default_rng(seed)
+    k, v = heads(rng, (ctx, n_kvh), hd=hd), heads(rng, (ctx, n_kvh), hd=hd)
+    q = heads(rng, (n_tok, n_head), hd=hd)
+    return k, v, q, rng.standard_normal(q.shape).astype(np.float32)
+
+
+# (kind, n_head, n_kvh, hd, n_tok, base, max_kv below base + n_tok, shift)
+CASES = [
+    (2, 24, 2, 256, 301, 640, 0, 0),    # 28.2 tiles, unsplit and split
+    (2, 24, 2, 256, 700, 0, 0, 0),      # causal from position 0: the last tiles split
+    (1, 16, 2, 256, 130, 1999, 0, 0),   # f16
+    (2, 8, 2, 256, 600, 700, 0, 1),     # 4 heads per KV head, unaligned queries
+    (2, 20, 1, 256, 9, 33, 0, 0),       # more than 16 heads per KV head
+    (2, 16, 2, 256, 280, 1000, 150, 0), # the cache ends before the tokens do
+    (1, 32, 8, 128, 33, 95, 0, 0),      # 128 dims, 64 positions per pass
+    (2, 32, 8, 128, 1, 5000, 0, 0),     # one token, many splits
+    (2, 3, 1, 128, 65, 62, 40, 3),      # KV rows of 136 bytes
+    (1, 24, 8, 64, 43, 127, 0, 0),      # 64 dims, 128 positions per pass
+    (2, 16, 4, 64, 2, 0, 0, 0),         # the smallest prompt
+    (2, 4, 4, 64, 129, 3000, 0, 0),     # one head per KV head
+]
+
+
+@pytest.mark.parametrize("kind,n_head,n_kvh,hd,n_tok,base,cut,shift", CASES)
+def test_dense_prefill(rt, oracle, kind, n_head, n_kvh, hd, n_tok, base, cut, shift):
+    note(f"dense kind={kind} heads={n_head}/{n_kvh} hd={hd} n_tok={n_tok} base={base} cut={cut}")
+    ctx = base + n_tok
+    k, v, q, gate = _inputs(31 * hd + n_tok, kind, n_head, n_kvh, hd, n_tok, ctx)
+    kc, _ = quantize_on_gpu(rt, k, kind)
+    vc, _ = quantize_on_gpu(rt, v, kind)
+    got = _run(rt, q, gate, kc, vc, kind, n_kvh, base, ctx - cut, shift)
+    want = oracle.attn(q, oracle.encode(k, kind), oracle.encode(v, kind), kind, n_head, n_kvh, hd,
+                       n_tok, gate=gate, kv_base=base, max_kv=ctx - cut, threads=8)
+    assert_attn_close(got, want, what=f"dense hd={hd} gqa={n_head // n_kvh}")
+    for p in (kc, vc):
+        rt.free(p)
+
+
+@pytest.mark.parametrize("kind,hd", [(2, 128), (1, 128), (1, 64), (2, 256)])
+def test_values_not_finite(rt, kind, hd):
+    """inf / NaN in one V row: tokens that do not see it are bit-identical to
+    the call without it, the others are not finite in exactly its dims (NaN, or
+    inf where both parts of a weight have one sign)."""
+    n_head, n_kvh, n_tok, base = 16, 2, 300, 1500
+    note(f"dense V not finite kind={kind} hd={hd}")
+    ctx, bad, kh = base + n_tok, base + 170, 1
+    k, v, q, gate = _inputs(5 + hd, kind, n_head, n_kvh, hd, n_tok, ctx)
+    kc, _ = quantize_on_gpu(rt, k, kind)
+    vc, nb = quantize_on_gpu(rt, v, kind)
+    clean = _run(rt, q, gate, kc, vc, kind, n_kvh, base, ctx)
+    rows = rt.download(vc, nb).reshape(ctx, n_kvh, -1).copy()
+    if kind == q4kv.KV_Q8:  # the scale of the row's second block
+        rows[bad, kh].view(np.uint16)[17] = 0x7C00
+        dims = np.arange(32, 64)
+    else:
+        rows[bad, kh].view(np.uint16)[[3, 40]] = (0x7E00, 0xFC00)
+        dims = np.array([3, 40])
+    rt.h2d(vc, rows)
+    got = _run(rt, q, gate, kc, vc, kind, n_kvh, base, ctx)
+    hit = np.zeros(q.shape, bool)
+    hit[bad - base:, kh * n_head // n_kvh:, dims] = True
+    assert not np.isfinite(got[hit]).any()
+    assert np.array_equal(got[~hit], clean[~hit])
+    for p in (kc, vc):
+        rt.free(p)
