@@ -4,7 +4,7 @@
  * The dense half of the reference's prefill kernel (gqa_prefill_k,
  * src/q4_rocm.cu:7020-7205): token t of n_tok attends positions
  * 0 .. min(kv_base + t + 1, max_kv) - 1 of a q8_0 or f16 cache,
- *   out = softmax(scale * q.k) v * sigmoid(gate).
+ *   out = softmax(scale * q.k) v * q4kv_sigmoid(gate).
  *
  * Consecutive tokens see nearly the same positions, so the tokens and the
  * query heads of one KV head are the columns of one matrix product: column
@@ -87,19 +87,6 @@ __device__ inline float col_max(float v) {
 __device__ inline float col_sum(float v) {
     v += __shfl_xor(v, 16);
     return v + __shfl_xor(v, 32);
-}
-
-/* 1 / (1 + e^-g) within 2 ulp: e^-g as 2^t with the product's rounding error
- * put back, and a reciprocal with one Newton step (a wave forms 64 of these
- * per lane: expf and the IEEE division took 5 us of a workgroup's end). */
-__device__ inline float sigmoid(float g) {
-    const float x = __builtin_amdgcn_fmed3f(g, -88.f, 88.f); /* e^88 is finite */
-    const float t = x * -1.44269502f;
-    const float lo = fmaf(x, -1.92596303e-8f, fmaf(x, -1.44269502f, -t));
-    const float e = __builtin_amdgcn_exp2f(t);
-    const float d = 1.f + fmaf(e, lo * 0.693147182f, e);
-    const float r = __builtin_amdgcn_rcpf(d);
-    return g == g ? fmaf(fmaf(-d, r, 1.f), r, r) : g;
 }
 
 /* Four biased bytes (w ^ 0x80..) -> 1024 + u in four fp16. */
@@ -550,7 +537,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
             const f4_t g = ldg((const f4_t *)(a.gate + ro + 16u * T));
             f4_t r;
 #pragma unroll
-            for (uint32_t i = 0; i < 4u; i++) r[i] = acc[T][i] * inv * sigmoid(g[i]);
+            for (uint32_t i = 0; i < 4u; i++) r[i] = acc[T][i] * inv * q4kv_sigmoid(g[i]);
             stg((f4_t *)(a.out + ro + 16u * T), r);
         }
     } else {
@@ -559,7 +546,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
 #pragma unroll
             for (uint32_t i = 0; i < 4u; i++)
                 stg(a.out + ro + 16u * T + i,
-                    acc[T][i] * inv * sigmoid(ldg(a.gate + ro + 16u * T + i)));
+                    acc[T][i] * inv * q4kv_sigmoid(ldg(a.gate + ro + 16u * T + i)));
     }
 }
 
@@ -607,7 +594,7 @@ template <int HD> __global__ __launch_bounds__(256) void qsa_dense_merge_k(Args 
 #pragma unroll
     for (uint32_t k = 0; k < 4u; k++) {
         const float r = L > 0.f ? acc[k] / L : 0.f;
-        stg(a.out + ro + k, r * sigmoid(g[k]));
+        stg(a.out + ro + k, r * q4kv_sigmoid(g[k]));
     }
 }
 
@@ -689,18 +676,20 @@ bool q4kv_dense_takes(int kind, uint32_t hd, uint32_t n_tok, uint32_t n_kvh, uin
     if ((cols / COLS + 1u) * n_kvh >= 0x1000000u) return false;
     static const char *force = getenv("Q4KV_DENSE"); /* 0: never, 1: every shape it can */
     if (force) return force[0] != '0';
-    /* 64 and 128 dims, or more heads than the other kernels tile: at any
-     * size (the general kernels take 1.3 to 70 times as long from one token
-     * on). 256 dims: where the chunk, slab and f16 kernels' row slots (KV
-     * heads x head groups x attended positions) pass 280 thousand: a launch
-     * costs this kernel ~13 us however small, 20-25 us of work of theirs
-     * (24 / 2 heads, 64 tokens: 22.9 against 21.6 us over 300 positions,
-     * 29.3 against 34.7 over 1000; 16 / 2 heads, 64 tokens: 27.6 against
-     * 23.8 over 1000, 37.3 against 46.7 over 4000). */
-    if (hd != 256u || gqa > 16u) return true;
+    /* More heads than the other kernels tile: at any size (the general
+     * kernel takes 1.3 to 70 times as long). Otherwise where the other
+     * kernels' row slots (KV heads x head groups x attended positions) pass
+     * a limit: a launch costs this kernel 7 to 13 us however small.
+     * 256 dims, 280 thousand: 24 / 2 heads, 64 tokens: 22.9 against 21.6 us
+     * over 300 positions, 29.3 against 34.7 over 1000; 16 / 2 heads, 64
+     * tokens: 27.6 against 23.8 over 1000, 37.3 against 46.7 over 4000.
+     * 64 and 128 dims (q4kv_rows.hip), 160 thousand: 32 / 8 heads of 128
+     * dims: 13.6 against 12.1 us for 8 tokens over 1000 positions, 30.7
+     * against 32.1 for 2 over 16000, 32.0 against 86.9 for 8. */
+    if (gqa > 16u) return true;
     const uint64_t slots = (uint64_t)n_tok * n_kvh * (gqa > 8u ? 2u : 1u) *
                            (max_n - std::min<uint64_t>(max_n, n_tok) / 2u);
-    return n_tok > 1u && slots > 280000u;
+    return n_tok > 1u && slots > (hd == 256u ? 280000u : 160000u);
 }
 
 bool q4kv_dense_launch(int kind, uint32_t hd, const float *q, const void *kc, const void *vc,

@@ -167,6 +167,19 @@ __device__ static inline void q4kv_app_wg(const q4kv_app_args &a, uint32_t w) {
  * hold: returns the number of extra workgroups it needs (0: none held). */
 uint32_t q4kv_take_held(q4kv_app_args *a);
 
+/* 1 / (1 + e^-g) within 2 ulp: e^-g as 2^t with the product's rounding error
+ * put back, and a reciprocal with one Newton step (a wave forms 64 of these
+ * per lane: expf and the IEEE division took 5 us of a workgroup's end). */
+__device__ static inline float q4kv_sigmoid(float g) {
+    const float x = __builtin_amdgcn_fmed3f(g, -88.f, 88.f); /* e^88 is finite */
+    const float t = x * -1.44269502f;
+    const float lo = fmaf(x, -1.92596303e-8f, fmaf(x, -1.44269502f, -t));
+    const float e = __builtin_amdgcn_exp2f(t);
+    const float d = 1.f + fmaf(e, lo * 0.693147182f, e);
+    const float r = __builtin_amdgcn_rcpf(d);
+    return g == g ? fmaf(fmaf(-d, r, 1.f), r, r) : g;
+}
+
 /* ---- shared wave-level arithmetic of the Q/K preparation ---- */
 template <int CTRL> __device__ static inline float q4kv_dpp(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
