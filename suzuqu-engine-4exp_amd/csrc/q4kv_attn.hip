@@ -2365,434 +2365,6 @@ __global__ __launch_bounds__(256, 2) void qsa_f32w_k(AttnArgs a) {
     }
 }
 
-/* ------------------------------------------------------------------------
- * Prefill band kernel: the recent window that consecutive prefill tokens'
- * lists share, as dense MFMA tiles. A token's band is the longest run of
- * consecutive positions that ends its list (the causal recent window); the
- * slab kernel then attends only the list entries before it. One workgroup
- * takes BAND_TOK consecutive tokens of one KV head (two per wave): the union
- * of their bands (at most BAND_SPAN positions) streams through LDS 32
- * positions per pass (two passes in flight), where the workgroup dequantises
- * the K and V rows once into fp16 hi + lo parts (k * scale, exact to
- * ~2^-22), shared by every token and head of the tile. Each wave then runs,
- * for its two tokens with every LDS operand read once for both,
- *   S^T = K' Q^T   (A = K' hi / lo rows, B = a token's Q^T, columns 0-7 the
- *                   fp16 part of 8 heads' q, 8-15 the residual),
- *   softmax over the token's band positions only (the rest -inf),
- *   O^T += V'^T P^T (A = V'^T hi / lo, B = the weights split hi / lo),
- * with no per-position scale work on the VALU. The result is the (m, l,
- * unnormalised acc) partial of each (token, head), handed to the slab
- * kernel's final merge.
- * ------------------------------------------------------------------------ */
-constexpr uint32_t BAND_TPW = 2;                /* tokens per wave */
-constexpr uint32_t BAND_WAVES = 8;              /* waves per workgroup */
-constexpr uint32_t BAND_TOK = BAND_WAVES * BAND_TPW; /* tokens per workgroup */
-constexpr uint32_t BAND_MIN = 64;               /* shortest run worth a band */
-constexpr uint32_t BAND_SPAN = 1024;            /* widest union of a workgroup's bands */
-constexpr uint32_t BP = 32;                     /* positions per pass */
-
-/* workgroup barrier that waits for this wave's LDS accesses only (the
- * __syncthreads fence also drains every outstanding global load, including
- * the next pass's DMA) */
-__device__ static inline void barrier_lds(void) {
-    __builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0) */
-    __builtin_amdgcn_s_barrier();
-}
-
-/* The band of one token's list (wave-uniform): the run of consecutive
- * positions that ends it (after any padding), at least BAND_MIN long.
- * Returns the list index where the run starts (width if there is none) and
- * the run's first and last positions (ps > pe if none). */
-__device__ static inline uint32_t band_of(const int32_t *list, uint32_t width, uint32_t max_kv,
-                                          uint32_t lane, int32_t &ps, int32_t &pe) {
-    ps = 1;
-    pe = 0;
-    int32_t e = -1, vend = 0;
-    for (int32_t base = (int32_t)width - 64;; base -= 64) {
-        const int32_t j = base + (int32_t)lane;
-        const int32_t v = j >= 0 ? ldg(list + j) : -1;
-        const bool ok = j >= 0 && v >= 0 && (uint32_t)v < max_kv;
-        const uint64_t bal = __ballot(ok);
-        if (bal) {
-            const uint32_t hi = 63u - (uint32_t)__builtin_clzll(bal);
-            e = base + (int32_t)hi;
-            vend = __shfl(v, (int)hi);
-            break;
-        }
-        if (base <= 0) break;
-    }
-    if (e < 0) return width;
-    uint32_t run = 0;
-    for (uint32_t w0 = 0; w0 < BAND_SPAN; w0 += 64u) {
-        const int32_t j = e - (int32_t)(w0 + lane);
-        const bool ok = j >= 0 && ldg(list + j) == vend - (int32_t)(w0 + lane);
-        const uint64_t bad = __ballot(!ok);
-        if (bad) {
-            run = w0 + (uint32_t)__builtin_ctzll(bad);
-            break;
-        }
-        run = w0 + 64u;
-    }
-    /* a run stops at position 0 (a -1 entry before it equals vend - run too) */
-    if ((int64_t)run > (int64_t)vend + 1) run = (uint32_t)vend + 1u;
-    if (run > BAND_SPAN) run = BAND_SPAN;
-    if (run < BAND_MIN) return width;
-    ps = vend - (int32_t)run + 1;
-    pe = vend;
-    return (uint32_t)(e - (int32_t)run + 1);
-}
-
-/* band_of with every load issued at once: the last BAND_NJ x 64 entries of
- * the list (one load per lane each) cover the run whenever the list's last
- * valid entry is among its final 64 (no more than 63 trailing padding or
- * out-of-range entries); otherwise the chained band_of runs. Same result. */
-constexpr uint32_t BAND_NJ = BAND_SPAN / 64u + 1u;
-__device__ static inline uint32_t band_of_tail(const int32_t *list, uint32_t width,
-                                               uint32_t max_kv, uint32_t lane, int32_t &ps,
-                                               int32_t &pe) {
-    int32_t v[BAND_NJ];
-#pragma unroll
-    for (uint32_t i = 0; i < BAND_NJ; i++) {
-        const uint32_t j = 64u * i + lane; /* entry width - 1 - j */
-        v[i] = j < width ? ldg(list + (width - 1u - j)) : -1;
-    }
-    /* the last valid entry: the smallest j with a valid position */
-    const uint64_t okb = __ballot(v[0] >= 0 && (uint32_t)v[0] < max_kv);
-    if (!okb) return band_of(list, width, max_kv, lane, ps, pe);
-    const uint32_t jf = (uint32_t)__builtin_ctzll(okb);
-    const int32_t vend = __shfl(v[0], (int)jf);
-    /* the run: entry width - 1 - j holds vend - (j - jf) for j = jf, jf + 1, .. */
-    uint32_t run = BAND_NJ * 64u - jf; /* every loaded entry from jf on matches */
-#pragma unroll
-    for (uint32_t i = 0; i < BAND_NJ; i++) {
-        const uint32_t j = 64u * i + lane;
-        const bool bad = j >= jf && (j >= width || v[i] != vend - (int32_t)(j - jf));
-        const uint64_t bb = __ballot(bad);
-        if (bb) {
-            run = min(run, 64u * i + (uint32_t)__builtin_ctzll(bb) - jf);
-            break;
-        }
-    }
-    ps = 1;
-    pe = 0;
-    /* a run stops at position 0 (a -1 entry before it equals vend - run too) */
-    if ((int64_t)run > (int64_t)vend + 1) run = (uint32_t)vend + 1u;
-    if (run > BAND_SPAN) run = BAND_SPAN;
-    if (run < BAND_MIN) return width;
-    ps = vend - (int32_t)run + 1;
-    pe = vend;
-    return width - 1u - jf - run + 1u;
-}
-
-__global__ __launch_bounds__(512, 2) void qsa_band_k(AttnArgs a) {
-    constexpr uint32_t ROWB = 272, NCH = 17, KPAD = 264, VPAD = 40, TW = BAND_TPW;
-    /* K rows | V rows of even and odd passes: two passes in flight (two
-     * objects, so the LDS-DMA wait before reading one buffer does not cover
-     * the other's DMA) */
-    __shared__ __attribute__((aligned(16))) uint8_t rawA[2 * BP * ROWB];
-    __shared__ __attribute__((aligned(16))) uint8_t rawB[2 * BP * ROWB];
-    /* K' [hi/lo][position][dim] and V'^T [hi/lo][dim][slot] (fp16); V slot
-     * 8 g + i holds position 4 g + i (i < 4) or 16 + 4 g + i - 4, the
-     * positions a lane of k-group g holds in the score tiles */
-    __shared__ __attribute__((aligned(16))) _Float16 kp[2][BP][KPAD];
-    __shared__ __attribute__((aligned(16))) _Float16 vt[2][256][VPAD];
-    __shared__ int32_t s_ps[BAND_TOK], s_pe[BAND_TOK];
-
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t kh = blockIdx.y, t0 = blockIdx.x * BAND_TOK + wave * TW;
-    const uint32_t n_tok = a.kv_base; /* tokens of the launch (set by the host) */
-    const uint32_t gqa = a.n_head / a.n_kvh, width = a.width;
-    const uint32_t c = lane & 15u, jg = lane >> 4;
-    const float nsel = c >= 8u ? -1.f : 0.f;
-    const size_t rstride = (size_t)a.n_kvh * ROWB;
-    const uint8_t *kbase = a.kc + (size_t)kh * ROWB, *vbase = a.vc + (size_t)kh * ROWB;
-
-    TRACEB(0);
-    /* ---- the bands of this wave's tokens ---- */
-    int32_t ps[TW], pe[TW];
-    uint32_t nb[TW];
-#pragma unroll
-    for (uint32_t k = 0; k < TW; k++) {
-        const uint32_t t = t0 + k;
-        ps[k] = 1;
-        pe[k] = 0;
-        nb[k] = width;
-        if (t < n_tok)
-            nb[k] = band_of_tail(a.idx + (size_t)t * a.tok_stride + (size_t)kh * a.kvh_stride,
-                                 width, a.max_kv, lane, ps[k], pe[k]);
-        if (lane == 0) {
-            s_ps[wave * TW + k] = ps[k];
-            s_pe[wave * TW + k] = pe[k];
-        }
-    }
-    __syncthreads();
-    int32_t lo = INT32_MAX, hi = INT32_MIN;
-#pragma unroll
-    for (uint32_t w = 0; w < BAND_TOK; w++)
-        if (s_ps[w] <= s_pe[w]) {
-            lo = min(lo, s_ps[w]);
-            hi = max(hi, s_pe[w]);
-        }
-    const bool tile = lo <= hi && (int64_t)hi - lo + 1 <= (int64_t)BAND_SPAN;
-#pragma unroll
-    for (uint32_t k = 0; k < TW; k++) {
-        const uint32_t t = t0 + k;
-        if (!tile) {
-            ps[k] = 1;
-            pe[k] = 0;
-            nb[k] = width;
-        }
-        if (t < n_tok) {
-            const uint32_t item = t * a.n_kvh + kh;
-            if (lane == 0) a.band_nb[item] = (int32_t)nb[k];
-            if (ps[k] > pe[k] && lane < gqa)
-                stg((fv2 *)(a.band_ml + ((size_t)item * gqa + lane) * 2u), (fv2){-INFINITY, 0.f});
-        }
-    }
-    if (!tile) return; /* uniform over the workgroup */
-    TRACEB(1);
-    const uint32_t n_pass = (uint32_t)(hi - lo) / BP + 1u;
-
-    /* the Q^T operands of this wave's tokens, natural dim order. Each head's
-     * q x scale is divided by the power of two 2^e that brings its largest
-     * magnitude into [0.5, 1) (exact: the fp16 parts neither overflow nor
-     * lose relative precision), and its scores are multiplied by qmul = 2^e;
-     * the eight lanes holding a head (columns c, c + 8, k-groups 0-3) find
-     * its maximum together. */
-    h8_t qB[TW][8];
-    float qmul[TW];
-#pragma unroll
-    for (uint32_t k = 0; k < TW; k++) {
-        const uint32_t t = t0 + k, h = c & 7u;
-        const bool hv = t < n_tok && h < gqa;
-        const float *qr = a.q + ((size_t)(t < n_tok ? t : 0u) * a.n_head + kh * gqa + (hv ? h : 0u)) * 256u;
-        float am = 0.f;
-#pragma unroll
-        for (uint32_t b = 0; b < 8u; b++) {
-            const f4_t x0 = ldg((const f4_t *)(qr + 32u * b + 8u * jg));
-            const f4_t x1 = ldg((const f4_t *)(qr + 32u * b + 8u * jg + 4u));
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; i++) am = fmaxf(am, fmaxf(fabsf(x0[i]), fabsf(x1[i])));
-        }
-        am = fmaxf(am, __shfl_xor(am, 8));
-        am = fmaxf(am, __shfl_xor(am, 16));
-        am = fmaxf(am, __shfl_xor(am, 32));
-        am *= a.scale_log2;
-        const int e = (am > 0.f && am <= 3.4e38f) ? __builtin_amdgcn_frexp_expf(am) : 0;
-        qmul[k] = __builtin_ldexpf(1.f, e);
-        const float qs = hv ? __builtin_ldexpf(a.scale_log2, -e) : 0.f;
-#pragma unroll
-        for (uint32_t b = 0; b < 8u; b++) {
-            const f4_t x0 = ldg((const f4_t *)(qr + 32u * b + 8u * jg));
-            const f4_t x1 = ldg((const f4_t *)(qr + 32u * b + 8u * jg + 4u));
-            qB[k][b] = __builtin_bit_cast(
-                h8_t, (u4_t){split_pk(x0[0] * qs, x0[1] * qs, nsel), split_pk(x0[2] * qs, x0[3] * qs, nsel),
-                             split_pk(x1[0] * qs, x1[1] * qs, nsel), split_pk(x1[2] * qs, x1[3] * qs, nsel)});
-        }
-    }
-
-    /* the rows of pass p: 32 positions x 17 sixteen-byte pieces per cache;
-     * wave w issues K and V instruction w (and wave 0 / 1 the ninth) */
-    auto issue = [&](uint32_t pass, uint8_t *rawb) {
-        const int32_t base = lo + (int32_t)(pass * BP);
-        /* K and V instruction u = wave; wave 0 / 1 also the ninth K / V
-         * instruction */
-#pragma unroll
-        for (uint32_t k = 0; k < 2u; k++) {
-            const uint32_t u = k == 0u ? wave : 8u;
-            if (k == 1u && wave > 1u) break;
-            const uint32_t e = u * 64u + lane;
-            const uint32_t r = e / NCH, q = e - r * NCH;
-            int32_t p = base + (int32_t)r;
-            if (p > hi || (uint32_t)p >= a.max_kv) p = lo; /* outside every band: masked */
-            const size_t off = (size_t)p * rstride + q * 16u;
-            if (u < 8u || lane < 32u) {
-                if (k == 0u || wave == 0u) dma16_manual(kbase + off, rawb + u * 1024u);
-                if (k == 0u || wave == 1u) dma16_manual(vbase + off, rawb + BP * ROWB + u * 1024u);
-            }
-        }
-    };
-    /* the Q operands are complete before the first DMA: a compiler wait for
-     * a load issued after the (assembly) DMAs would drain those too */
-#pragma unroll
-    for (uint32_t k = 0; k < TW; k++)
-#pragma unroll
-        for (uint32_t bb = 0; bb < 8u; bb++) asm volatile("" ::"v"(qB[k][bb]));
-    TRACEB(2);
-    issue(0u, rawA);
-    if (n_pass > 1u) issue(1u, rawB);
-
-    float m_run[TW], l_run[TW];
-    f4_t acc[TW][16];
-#pragma unroll
-    for (uint32_t k = 0; k < TW; k++) {
-        m_run[k] = -INFINITY;
-        l_run[k] = 0.f;
-#pragma unroll
-        for (uint32_t T = 0; T < 16u; T++) acc[k][T] = (f4_t){0.f, 0.f, 0.f, 0.f};
-    }
-
-    auto run_pass = [&](uint32_t pass, uint8_t *rawb) {
-        /* this pass's rows landed (the next pass's may still be in flight:
-         * s_waitcnt vmcnt(n) with the lgkm / exp counts unconstrained; waves
-         * 0 and 1 issue three DMA instructions per pass, the others two) */
-        if (pass + 1u < n_pass) {
-            if (wave <= 1u)
-                __builtin_amdgcn_s_waitcnt(0x0F73);
-            else
-                __builtin_amdgcn_s_waitcnt(0x0F72);
-        } else {
-            __builtin_amdgcn_s_waitcnt(0);
-        }
-        barrier_lds(); /* rows landed; every wave done with the last pass */
-        if (pass == 4u) TRACEB(3);
-        /* ---- dequantise: K' rows (work item: position x >> 4, 16 dims) ---- */
-#pragma unroll
-        for (uint32_t x = tid; x < 512u; x += 64u * BAND_WAVES) {
-            const uint32_t p = x >> 4, d0 = 16u * (x & 15u), b = d0 >> 5;
-            const uint8_t *src = rawb + p * ROWB + 34u * b + 2u + (d0 & 31u);
-            const float ks = ld_h(rawb + p * ROWB + 34u * b);
-            uint32_t hw[8], lw[8];
-#pragma unroll
-            for (uint32_t i = 0; i < 8u; i++) {
-                const uint32_t w = *(const uint16_t *)(src + 2u * i);
-                const float x0 = (float)(int32_t)(int8_t)(w & 0xffu) * ks;
-                const float x1 = (float)(int32_t)(int8_t)(w >> 8) * ks;
-                hw[i] = pkrtz(x0, x1);
-                lw[i] = pkrtz(x0 - h2lo(hw[i]), x1 - h2hi(hw[i]));
-            }
-            *(u4_t *)&kp[0][p][d0] = (u4_t){hw[0], hw[1], hw[2], hw[3]};
-            *(u4_t *)&kp[0][p][d0 + 8u] = (u4_t){hw[4], hw[5], hw[6], hw[7]};
-            *(u4_t *)&kp[1][p][d0] = (u4_t){lw[0], lw[1], lw[2], lw[3]};
-            *(u4_t *)&kp[1][p][d0 + 8u] = (u4_t){lw[4], lw[5], lw[6], lw[7]};
-        }
-        /* ---- V'^T (work item: dims 2 dp, 2 dp + 1, slots 8 g .. 8 g + 7) ---- */
-#pragma unroll
-        for (uint32_t x = tid; x < 512u; x += 64u * BAND_WAVES) {
-            const uint32_t dp = x & 127u, g = x >> 7, b = dp >> 4;
-            const uint8_t *vr = rawb + BP * ROWB;
-            uint32_t he[4], le[4], ho[4], lo4[4];
-#pragma unroll
-            for (uint32_t i2 = 0; i2 < 4u; i2++) {
-                float xe[2], xo[2];
-#pragma unroll
-                for (uint32_t k = 0; k < 2u; k++) {
-                    const uint32_t i = 2u * i2 + k;
-                    const uint32_t p = i < 4u ? 4u * g + i : 16u + 4u * g + i - 4u;
-                    const uint8_t *row = vr + p * ROWB + 34u * b;
-                    const float vs = ld_h(row);
-                    const uint32_t w = *(const uint16_t *)(row + 2u + 2u * (dp & 15u));
-                    xe[k] = (float)(int32_t)(int8_t)(w & 0xffu) * vs;
-                    xo[k] = (float)(int32_t)(int8_t)(w >> 8) * vs;
-                }
-                he[i2] = pkrtz(xe[0], xe[1]);
-                le[i2] = pkrtz(xe[0] - h2lo(he[i2]), xe[1] - h2hi(he[i2]));
-                ho[i2] = pkrtz(xo[0], xo[1]);
-                lo4[i2] = pkrtz(xo[0] - h2lo(ho[i2]), xo[1] - h2hi(ho[i2]));
-            }
-            *(u4_t *)&vt[0][2u * dp][8u * g] = (u4_t){he[0], he[1], he[2], he[3]};
-            *(u4_t *)&vt[1][2u * dp][8u * g] = (u4_t){le[0], le[1], le[2], le[3]};
-            *(u4_t *)&vt[0][2u * dp + 1u][8u * g] = (u4_t){ho[0], ho[1], ho[2], ho[3]};
-            *(u4_t *)&vt[1][2u * dp + 1u][8u * g] = (u4_t){lo4[0], lo4[1], lo4[2], lo4[3]};
-        }
-        barrier_lds(); /* K', V'^T ready; this pass's raw rows are free */
-        if (pass == 4u) TRACEB(4);
-        if (pass + 2u < n_pass) issue(pass + 2u, rawb);
-        const int32_t base = lo + (int32_t)(pass * BP);
-        bool live[TW], any = false;
-#pragma unroll
-        for (uint32_t k = 0; k < TW; k++) {
-            live[k] = ps[k] <= pe[k] && base <= pe[k] && base + (int32_t)BP - 1 >= ps[k];
-            any = any || live[k];
-        }
-        if (!any) return; /* wave-uniform */
-        if (pass == 4u) TRACEB(5);
-        /* ---- scores of the tokens' 8 heads at the pass's 32 positions ---- */
-        f4_t S[TW][2];
-#pragma unroll
-        for (uint32_t k = 0; k < TW; k++) S[k][0] = S[k][1] = (f4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (uint32_t b = 0; b < 8u; b++) {
-#pragma unroll
-            for (uint32_t tt = 0; tt < 2u; tt++) {
-#pragma unroll
-                for (uint32_t hl = 0; hl < 2u; hl++) {
-                    const h8_t A = *(const h8_t *)&kp[hl][16u * tt + c][32u * b + 8u * jg];
-#pragma unroll
-                    for (uint32_t k = 0; k < TW; k++)
-                        S[k][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, qB[k][b], S[k][tt], 0, 0, 0);
-                }
-            }
-        }
-        h8_t B[TW];
-#pragma unroll
-        for (uint32_t k = 0; k < TW; k++) {
-            float T[8];
-#pragma unroll
-            for (uint32_t i = 0; i < 8u; i++) {
-                const int32_t P = base + (int32_t)((i < 4u ? 0u : 16u) + 4u * jg + (i & 3u));
-                const float x = add_ror8(S[k][i >> 2][i & 3u]) * qmul[k];
-                T[i] = (P >= ps[k] && P <= pe[k]) ? x : -INFINITY;
-            }
-            float mx = fmax3v(fmax3v(T[0], T[1], T[2]), fmax3v(T[3], T[4], T[5]), fmax2(T[6], T[7]));
-            mx = max32(max16(mx));
-            const float mn = fmax2(m_run[k], mx);
-            const float ms = mn == -INFINITY ? 0.f : mn;
-            const float alpha = __builtin_amdgcn_exp2f(m_run[k] - ms);
-            const bool grew = mn > m_run[k];
-            m_run[k] = mn;
-            float P[8], ls = 0.f;
-#pragma unroll
-            for (uint32_t i = 0; i < 8u; i++) {
-                P[i] = __builtin_amdgcn_exp2f(T[i] - ms);
-                ls += P[i];
-            }
-            l_run[k] = l_run[k] * alpha + ls;
-            if (__ballot(grew) != 0u) {
-#pragma unroll
-                for (uint32_t T2 = 0; T2 < 16u; T2++) acc[k][T2] *= alpha;
-            }
-            B[k] = __builtin_bit_cast(
-                h8_t, (u4_t){split_pk(P[0], P[1], nsel), split_pk(P[2], P[3], nsel),
-                             split_pk(P[4], P[5], nsel), split_pk(P[6], P[7], nsel)});
-        }
-#pragma unroll
-        for (uint32_t T2 = 0; T2 < 16u; T2++) {
-#pragma unroll
-            for (uint32_t hl = 0; hl < 2u; hl++) {
-                const h8_t A = *(const h8_t *)&vt[hl][16u * T2 + c][8u * jg];
-#pragma unroll
-                for (uint32_t k = 0; k < TW; k++)
-                    acc[k][T2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[k], acc[k][T2], 0, 0, 0);
-            }
-        }
-        TRACEB(8u + (pass < 7u ? pass : 7u));
-    };
-    for (uint32_t pass = 0; pass < n_pass; pass += 2u) {
-        run_pass(pass, rawA);
-        if (pass == 4u) TRACEB(6);
-        if (pass + 1u < n_pass) run_pass(pass + 1u, rawB);
-    }
-    TRACEB(7);
-    /* ---- the partials: (m, l) per head, unnormalised rows in out ---- */
-#pragma unroll
-    for (uint32_t k = 0; k < TW; k++) {
-        const uint32_t t = t0 + k;
-        if (t >= n_tok || ps[k] > pe[k]) continue;
-        const uint32_t item = t * a.n_kvh + kh;
-        const float lw = pair32_sum(sum16(l_run[k]));
-        if (lane < gqa) stg((fv2 *)(a.band_ml + ((size_t)item * gqa + lane) * 2u), (fv2){m_run[k], lw});
-        float *orow = a.out + ((size_t)t * a.n_head + kh * gqa) * 256u;
-#pragma unroll
-        for (uint32_t T2 = 0; T2 < 16u; T2++) {
-            f4_t v;
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; i++) v[i] = add_ror8(acc[k][T2][i]);
-            if (c < gqa) stg((f4_t *)(orow + (size_t)c * 256u + 16u * T2 + 4u * jg), v);
-        }
-    }
-}
-
 /* Merge the S split partials of one (item, head): weights 2^(m_s - M) over
  * splits with l_s > 0, then the sigmoid gate (src/q4_rocm.cu:6968-7013).
  * Thread c owns output column c. For S <= COMB_REG every partial load
@@ -3267,6 +2839,7 @@ struct Plan {
  * Q4KV_SLAB=0 turns the slab kernel off, Q4KV_SLAB=2 uses it everywhere
  * (A/B measurement). */
 #define SLAB_MAX_WG 16384u
+#define SLAB_SPLIT_WG 1024u /* workgroups a prefill-sized launch is split to */
 static int slab_mode(void) {
     static int v = -1;
     if (v < 0) {
@@ -3365,7 +2938,7 @@ static Plan plan_launch(uint32_t hd, uint32_t n_items, uint32_t max_n, uint32_t 
         if (!prefill_sized) {
             choose_split(n_items, s_full, gqa, have_part, cap, S, cps);
         } else {
-            S = n_items >= SLAB_MAX_WG ? 1u : SLAB_MAX_WG / n_items;
+            S = n_items >= SLAB_SPLIT_WG ? 1u : SLAB_SPLIT_WG / n_items;
             if (S < 1u) S = 1u;
             if (S > COMB_REG) S = COMB_REG; /* the merge's register path */
             const size_t per = (size_t)gqa * PSTRIDE;
@@ -3425,6 +2998,49 @@ static bool held_matches(const AttnArgs &a) {
            h.n == a.n_kvh * 256u && h.bpt == a.n_kvh * 272u;
 }
 
+/* Listed prefill (q8_0, hd 256) through q4kv_sparse.hip, which converts a
+ * row once for up to 16 heads. Lists below 256 entries are too few passes for
+ * its four waves (100 entries: 44 against 40 us for 512 tokens). 9-16 heads
+ * per KV head: from 60 thousand row slots (items x list), below which the
+ * chunk kernel's shorter chain wins (16 tokens, 24 / 2 heads: 22.5 against
+ * 24.8 us at 2051 entries, 20.5 against 18.2 at 1000; 512 tokens: 180 against
+ * 329 at 2051). Up to 8 heads the slab kernel converts a row once as well:
+ * this one wins while a launch is about one round of workgroups (256 tokens,
+ * 16 / 2 heads: 85 against 120 us; 512: 161 against 179; 128: 54 against 52;
+ * 1024: 310 against 295). */
+static bool sparse_takes(uint32_t n_items, uint32_t max_n, uint32_t gqa) {
+    static const char *e = getenv("Q4KV_SPARSE"); /* 0: never, 1: always (measurement) */
+    if (e) return e[0] != '0' && n_items < 0x1000000u;
+    if (max_n < 256u || n_items >= 0x1000000u) return false;
+    return gqa > 8u ? n_items > 16u && (uint64_t)n_items * max_n >= 60000u
+                    : n_items >= 384u && n_items < 1536u;
+}
+static bool launch_sparse(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t gqa, PartBuf pb) {
+    if (!a.kc || !a.vc || !a.q || !a.out || !q4kv_flush()) return false;
+    const uint32_t n_pass = (max_n + 31u) / 32u;
+    uint32_t S = n_items < 512u ? 512u / n_items : 1u; /* the resident workgroups once */
+    if (S > n_pass / 8u) S = n_pass / 8u;
+    if (S < 1u || !pb.ptr) S = 1u;
+    while (S > 1u && (size_t)n_items * S * gqa * PSTRIDE > pb.cap) S--;
+    a.S = S;
+    a.part = pb.ptr;
+    a.item0 = 0u;
+    a.band_nb = nullptr;
+    a.band_ml = nullptr;
+    /* the shared window apart: 1024 tokens, 24 / 2 heads: 329 against 344 us;
+     * 512: 198 against 180 */
+    if (S == 1u && n_items >= 2048u && band_enabled() && pb.ptr && q4kv_band_floats(n_items, gqa) <= pb.cap) {
+        if (!q4kv_band_launch(a, n_items, pb.ptr)) return false;
+    }
+    if (!q4kv_sparse_launch(a, n_items)) return false;
+    for (uint32_t i0 = 0; S > 1u && i0 < n_items; i0 += Q4KV_MAX_GRID_Y) {
+        a.item0 = i0;
+        const uint32_t ni = n_items - i0 < Q4KV_MAX_GRID_Y ? n_items - i0 : Q4KV_MAX_GRID_Y;
+        qsa_comb_k<Q4KV_F32, MODE_INDEXED><<<dim3(gqa, ni), 256, 0, q4kv_stream>>>(a);
+    }
+    return q4kv_launch_ok("qsa sparse merge");
+}
+
 template <int KIND, int MODE>
 static bool launch_kind(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t gqa,
                         const OutProj *op = nullptr, PartBuf pb = lib_part()) {
@@ -3447,6 +3063,11 @@ static bool launch_kind(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t g
             if (!q4kv_flush()) return false;
             return q4kv_rows_launch(KIND, MODE, a, n_items, max_n, pb.ptr, pb.cap);
         }
+    }
+    if constexpr (KIND == Q4KV_Q8 && MODE == MODE_INDEXED) {
+        const bool al = ((((uintptr_t)a.kc) | ((uintptr_t)a.vc)) & 15u) == 0u;
+        if (a.hd == 256u && gqa <= 16u && al && !op && sparse_takes(n_items, max_n, gqa))
+            return launch_sparse(a, n_items, max_n, gqa, pb);
     }
     if (any_shape(a.hd, gqa)) {
         if (!q4kv_flush()) return false;
@@ -3519,16 +3140,12 @@ static bool launch_kind(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t g
         a.band_nb = nullptr;
         a.band_ml = nullptr;
         if (MODE == MODE_INDEXED && KIND == Q4KV_Q8 && pl.slab && S == 1u && gqa <= 8u &&
-            band_enabled() && pb.ptr && (size_t)ni * (1u + 2u * gqa) <= pb.cap && ni % a.n_kvh == 0u) {
+            band_enabled() && pb.ptr && q4kv_band_floats(ni, gqa) <= pb.cap && ni % a.n_kvh == 0u) {
             AttnArgs ab = a;
-            ab.band_nb = (int32_t *)pb.ptr;
-            ab.band_ml = pb.ptr + ni;
-            ab.kv_base = ni / a.n_kvh; /* tokens */
             ab.idx = a.idx + (size_t)(i0 / a.n_kvh) * a.tok_stride;
             ab.q = a.q + (size_t)(i0 / a.n_kvh) * a.n_head * a.hd;
             ab.out = a.out + (size_t)(i0 / a.n_kvh) * a.n_head * a.hd;
-            qsa_band_k<<<dim3((ni / a.n_kvh + BAND_TOK - 1u) / BAND_TOK, a.n_kvh), 64u * BAND_WAVES, 0,
-                         q4kv_stream>>>(ab);
+            if (!q4kv_band_launch(ab, ni, pb.ptr)) return false;
             a.band_nb = ab.band_nb - i0; /* indexed by the launch's item */
             a.band_ml = ab.band_ml - (size_t)i0 * gqa * 2u;
         }

@@ -216,4 +216,17 @@ bool q4kv_rows_takes(int kind, uint32_t hd, uint32_t gqa, bool rows16);
 bool q4kv_rows_launch(int kind, int mode, const AttnArgs &a, uint32_t n_items, uint32_t max_n,
                       float *part, size_t cap);
 
+/* Listed attention of many items over a q8_0 cache, hd 256, up to 16 query
+ * heads per KV head (q4kv_sparse.hip): a.S splits of each list, partials in
+ * natural column order. */
+bool q4kv_sparse_launch(const AttnArgs &a, uint32_t n_items);
+
+/* The shared recent window of consecutive prefill tokens' lists (q8_0, hd
+ * 256; q4kv_dense.hip): each token's band of consecutive positions at its
+ * list's end is attended as dense tiles. Sets a.band_nb (list entries before
+ * the band) and a.band_ml ((m, l) per head), in part, and leaves the bands'
+ * unnormalised rows in a.out. */
+size_t q4kv_band_floats(uint32_t n_items, uint32_t gqa);
+bool q4kv_band_launch(AttnArgs &a, uint32_t n_items, float *part);
+
 #endif

@@ -45,20 +45,12 @@
 #include <algorithm>
 #include <cmath>
 
-#include "q4kv_internal.h"
-
-extern "C" {
-#include "q4kv.h"
-}
+#include "q4kv_attn_item.h"
 
 namespace {
 
-typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef short s4_t __attribute__((ext_vector_type(4)));
-typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef float f2_t __attribute__((ext_vector_type(2)));
-typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr uint32_t NWAVE = 8, NTHR = 64 * NWAVE, COLS = 16 * NWAVE;
@@ -69,8 +61,6 @@ constexpr uint32_t PHEAD = 4; /* a partial row: m, l, two unused floats, HD accu
 __device__ inline uint32_t pk(float x, float y) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){x, y}, h2_t));
 }
-__device__ inline float h2lo(uint32_t w) { return (float)__builtin_bit_cast(h2_t, w)[0]; }
-__device__ inline float h2hi(uint32_t w) { return (float)__builtin_bit_cast(h2_t, w)[1]; }
 /* max of non-NaN operands, without fmaxf's canonicalisations */
 __device__ inline float max2(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, INFINITY); }
 
@@ -96,6 +86,95 @@ __device__ inline void biased_h4(uint32_t w, h2_t &lo, h2_t &hi) {
     hi = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w, 0x04030402u));
 }
 
+constexpr uint32_t BAND_MIN = 64;    /* shortest run worth a band */
+constexpr uint32_t BAND_SPAN = 1024; /* widest union of a workgroup's bands */
+constexpr uint32_t BAND_TOKS = 32;   /* most tokens per workgroup */
+
+/* The band of one token's list (wave-uniform): the run of consecutive
+ * positions that ends it (after any padding), at least BAND_MIN long.
+ * Returns the list index where the run starts (width if there is none) and
+ * the run's first and last positions (ps > pe if none). */
+__device__ inline uint32_t band_of(const int32_t *list, uint32_t width, uint32_t max_kv,
+                                          uint32_t lane, int32_t &ps, int32_t &pe) {
+    ps = 1;
+    pe = 0;
+    int32_t e = -1, vend = 0;
+    for (int32_t base = (int32_t)width - 64;; base -= 64) {
+        const int32_t j = base + (int32_t)lane;
+        const int32_t v = j >= 0 ? ldg(list + j) : -1;
+        const bool ok = j >= 0 && v >= 0 && (uint32_t)v < max_kv;
+        const uint64_t bal = __ballot(ok);
+        if (bal) {
+            const uint32_t hi = 63u - (uint32_t)__builtin_clzll(bal);
+            e = base + (int32_t)hi;
+            vend = __shfl(v, (int)hi);
+            break;
+        }
+        if (base <= 0) break;
+    }
+    if (e < 0) return width;
+    uint32_t run = 0;
+    for (uint32_t w0 = 0; w0 < BAND_SPAN; w0 += 64u) {
+        const int32_t j = e - (int32_t)(w0 + lane);
+        const bool ok = j >= 0 && ldg(list + j) == vend - (int32_t)(w0 + lane);
+        const uint64_t bad = __ballot(!ok);
+        if (bad) {
+            run = w0 + (uint32_t)__builtin_ctzll(bad);
+            break;
+        }
+        run = w0 + 64u;
+    }
+    /* a run stops at position 0 (a -1 entry before it equals vend - run too) */
+    if ((int64_t)run > (int64_t)vend + 1) run = (uint32_t)vend + 1u;
+    if (run > BAND_SPAN) run = BAND_SPAN;
+    if (run < BAND_MIN) return width;
+    ps = vend - (int32_t)run + 1;
+    pe = vend;
+    return (uint32_t)(e - (int32_t)run + 1);
+}
+
+/* band_of with every load issued at once: the last BAND_NJ x 64 entries of
+ * the list (one load per lane each) cover the run whenever the list's last
+ * valid entry is among its final 64 (no more than 63 trailing padding or
+ * out-of-range entries); otherwise the chained band_of runs. Same result. */
+constexpr uint32_t BAND_NJ = BAND_SPAN / 64u + 1u;
+__device__ inline uint32_t band_of_tail(const int32_t *list, uint32_t width,
+                                               uint32_t max_kv, uint32_t lane, int32_t &ps,
+                                               int32_t &pe) {
+    int32_t v[BAND_NJ];
+#pragma unroll
+    for (uint32_t i = 0; i < BAND_NJ; i++) {
+        const uint32_t j = 64u * i + lane; /* entry width - 1 - j */
+        v[i] = j < width ? ldg(list + (width - 1u - j)) : -1;
+    }
+    /* the last valid entry: the smallest j with a valid position */
+    const uint64_t okb = __ballot(v[0] >= 0 && (uint32_t)v[0] < max_kv);
+    if (!okb) return band_of(list, width, max_kv, lane, ps, pe);
+    const uint32_t jf = (uint32_t)__builtin_ctzll(okb);
+    const int32_t vend = __shfl(v[0], (int)jf);
+    /* the run: entry width - 1 - j holds vend - (j - jf) for j = jf, jf + 1, .. */
+    uint32_t run = BAND_NJ * 64u - jf; /* every loaded entry from jf on matches */
+#pragma unroll
+    for (uint32_t i = 0; i < BAND_NJ; i++) {
+        const uint32_t j = 64u * i + lane;
+        const bool bad = j >= jf && (j >= width || v[i] != vend - (int32_t)(j - jf));
+        const uint64_t bb = __ballot(bad);
+        if (bb) {
+            run = min(run, 64u * i + (uint32_t)__builtin_ctzll(bb) - jf);
+            break;
+        }
+    }
+    ps = 1;
+    pe = 0;
+    /* a run stops at position 0 (a -1 entry before it equals vend - run too) */
+    if ((int64_t)run > (int64_t)vend + 1) run = (uint32_t)vend + 1u;
+    if (run > BAND_SPAN) run = BAND_SPAN;
+    if (run < BAND_MIN) return width;
+    ps = vend - (int32_t)run + 1;
+    pe = vend;
+    return width - 1u - jf - run + 1u;
+}
+
 struct Args {
     const uint8_t *kc, *vc;
     const float *q, *gate;
@@ -105,6 +184,13 @@ struct Args {
      * the unsplit tiles T1 - 1 .. T2, the split ones, the tiles below T2 */
     uint32_t S, T1, T2;
     float scale_log2;
+    /* the band form (qsa_dense_k with BAND): lists, tokens per tile, and per
+     * item the entries before its band and the band's (m, l) per head */
+    const int32_t *idx;
+    uint64_t tok_stride, kvh_stride;
+    uint32_t width, toks;
+    int32_t *band_nb;
+    float *band_ml;
 };
 
 /* One pass's tile geometry. 256 threads hold one 32-value q8_0 block of K
@@ -128,7 +214,14 @@ template <uint32_t VS> __device__ inline uint32_t vaddr(uint32_t p, uint32_t pc)
     return p * VS + (((pc >> 1) ^ x) << 5) + (((pc ^ (p >> 3)) & 1u) << 4);
 }
 
-template <int KIND, int HD>
+/* BAND: listed prefill's shared part. A token's band is the longest run of
+ * consecutive positions that ends its list (the causal recent window, which
+ * consecutive tokens share); the tile's columns then see the positions of
+ * their own bands only, out of the union of the tile's bands, and leave
+ * (m, l) and unnormalised rows (in out) for the kernel that attends the list
+ * entries before the bands. A tile is whole tokens. Without a band for some
+ * token, or with a union past BAND_SPAN, the list is left as it is. */
+template <int KIND, int HD, bool BAND = false>
 __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     using G = Geo<KIND, HD>;
     constexpr uint32_t NB = G::NB, PT = G::PT, NT = G::NT, KG = G::KG, KS = G::KS, VS = G::VS;
@@ -162,18 +255,69 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     kh %= a.n_kvh;
     const uint32_t gqa = a.gqa;
     /* this lane's column */
-    const uint32_t col = tile * COLS + wave * 16u + c;
-    const bool live = col < a.n_tok * gqa;
-    const uint32_t t = live ? col / gqa : 0u, h = live ? col - t * gqa : 0u;
-    auto seen = [&](uint32_t tok) { /* positions token tok attends */
-        const uint64_t n = (uint64_t)a.kv_base + tok + 1u;
-        return n < a.max_kv ? (uint32_t)n : a.max_kv;
+    const uint32_t lc = wave * 16u + c, col = tile * COLS + lc;
+    const uint32_t t_in = BAND ? lc / gqa : 0u;
+    const bool live = BAND ? t_in < a.toks && tile * a.toks + t_in < a.n_tok : col < a.n_tok * gqa;
+    const uint32_t t = !live ? 0u : BAND ? tile * a.toks + t_in : col / gqa;
+    const uint32_t h = !live ? 0u : BAND ? lc - t_in * gqa : col - t * gqa;
+    /* the column sees positions lo_c .. n_c - 1, the workgroup's columns
+     * together lo_all .. n_all - 1, and all of them lo_max .. n_min - 1 */
+    uint32_t lo_c = 0u, n_c, lo_all = 0u, n_all, lo_max = 0u, n_min;
+    if constexpr (BAND) {
+        __shared__ int32_t s_lo[BAND_TOKS], s_hi[BAND_TOKS]; /* first and last position, hi < lo: none */
+        __shared__ uint32_t s_nb[BAND_TOKS];
+        for (uint32_t k = wave; k < a.toks; k += NWAVE) {
+            const uint32_t tk = tile * a.toks + k;
+            int32_t ps = 1, pe = 0;
+            uint32_t nb = a.width;
+            if (tk < a.n_tok)
+                nb = band_of_tail(a.idx + (size_t)tk * a.tok_stride + (size_t)kh * a.kvh_stride, a.width,
+                                  a.max_kv, lane, ps, pe);
+            if (lane == 0u) {
+                s_lo[k] = ps;
+                s_hi[k] = pe;
+                s_nb[k] = nb;
+            }
+        }
+        __syncthreads();
+        int32_t lo = INT32_MAX, hi = INT32_MIN, lom = 0, him = INT32_MAX;
+        for (uint32_t k = 0; k < a.toks && tile * a.toks + k < a.n_tok; k++) {
+            const bool has = s_lo[k] <= s_hi[k];
+            lo = has ? min(lo, s_lo[k]) : lo;
+            hi = has ? max(hi, s_hi[k]) : hi;
+            lom = max(lom, has ? s_lo[k] : 0);
+            him = min(him, has ? s_hi[k] : -1);
+        }
+        const bool use = lo <= hi && (int64_t)hi - lo + 1 <= (int64_t)BAND_SPAN;
+        if (tid < a.toks && tile * a.toks + tid < a.n_tok) {
+            const uint32_t item = (tile * a.toks + tid) * a.n_kvh + kh;
+            a.band_nb[item] = (int32_t)(use ? s_nb[tid] : a.width);
+            if (!use || s_lo[tid] > s_hi[tid])
+                for (uint32_t g = 0; g < gqa; g++)
+                    stg((f2_t *)(a.band_ml + ((size_t)item * gqa + g) * 2u), (f2_t){-INFINITY, 0.f});
+        }
+        if (!use) return; /* uniform over the workgroup */
+        lo_all = (uint32_t)lo;
+        n_all = (uint32_t)hi + 1u;
+        lo_max = (uint32_t)lom;
+        n_min = (uint32_t)(him + 1);
+        lo_c = live ? (uint32_t)s_lo[t_in] : 0u;
+        n_c = live ? (uint32_t)(s_hi[t_in] + 1) : 0u; /* none: 1 .. 0, nothing */
+    } else {
+        auto seen = [&](uint32_t tok) { /* positions token tok attends */
+            const uint64_t n = (uint64_t)a.kv_base + tok + 1u;
+            return n < a.max_kv ? (uint32_t)n : a.max_kv;
+        };
+        n_c = live ? seen(t) : 0u;
+        const uint32_t c_last = min((tile + 1u) * COLS, a.n_tok * gqa) - 1u;
+        n_all = seen(c_last / gqa);       /* of the workgroup's last token */
+        n_min = seen(tile * COLS / gqa);  /* of its first */
+    }
+    auto sees = [&](uint32_t p) { return p < n_c && (!BAND || p >= lo_c); };
+    auto partly = [&](uint32_t base) { /* some column does not see all of the pass */
+        return base + PT > n_min || (BAND && base < lo_max);
     };
-    const uint32_t n_c = live ? seen(t) : 0u;
-    const uint32_t c_last = min((tile + 1u) * COLS, a.n_tok * gqa) - 1u;
-    const uint32_t n_all = seen(c_last / gqa);         /* of the workgroup's last token */
-    const uint32_t n_min = seen(tile * COLS / gqa);    /* of its first */
-    const uint32_t n_pass = (n_all + PT - 1u) / PT;
+    const uint32_t n_pass = (n_all - lo_all + PT - 1u) / PT;
     const uint32_t p0 = (uint32_t)((uint64_t)n_pass * s / S);
     const uint32_t p1 = (uint32_t)((uint64_t)n_pass * (s + 1u) / S);
     if (tid < 2u) s_bad[tid] = 0u;
@@ -192,7 +336,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     u4_t rk[2], rv[2]; /* f16 */
     auto load = [&](uint32_t pass) {
         if constexpr (KIND == Q4KV_Q8) {
-            const uint32_t p = min(pass * PT + bp, n_all - 1u);
+            const uint32_t p = min(lo_all + pass * PT + bp, n_all - 1u);
             const uint8_t *src = (is_v ? vb : kb) + (size_t)p * rstride + 68u * (bb >> 1) + 32u * (bb & 1u);
             r0 = *(const GLOBAL u4u_t *)src;
             r1 = *(const GLOBAL u4u_t *)(src + 16);
@@ -201,7 +345,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
 #pragma unroll
             for (uint32_t i = 0; i < 2u; i++) {
                 const uint32_t e = tid + NTHR * i, pc = e % (HD / 8u);
-                const uint32_t p = min(pass * PT + e / (HD / 8u), n_all - 1u);
+                const uint32_t p = min(lo_all + pass * PT + e / (HD / 8u), n_all - 1u);
                 rk[i] = ldg((const u4_t *)(kb + (size_t)p * rstride) + pc);
                 rv[i] = ldg((const u4_t *)(vb + (size_t)p * rstride) + pc);
             }
@@ -209,7 +353,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     };
     auto store = [&](uint32_t pass) {
         const uint32_t buf = pass & 1u;
-        const bool masked = pass * PT + PT > n_min;
+        const bool masked = partly(lo_all + pass * PT);
         if constexpr (KIND == Q4KV_Q8) {
             const uint32_t d[9] = {r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3], r2};
             /* even blocks: the scale leads the first dword; odd blocks: it
@@ -331,8 +475,8 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     __syncthreads();
 
     for (uint32_t pass = p0; pass < p1; pass++) {
-        const uint32_t buf = pass & 1u, base = pass * PT;
-        const bool masked = base + PT > n_min; /* some column does not see all */
+        const uint32_t buf = pass & 1u, base = lo_all + pass * PT;
+        const bool masked = partly(base);
         if (masked && s_bad[buf] == pass + 1u) {
             /* Rows that not every column sees hold inf or NaN, which a zero
              * weight would turn into NaN. They are taken out of the tile,
@@ -354,7 +498,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
             }
             __syncthreads();
             for (uint32_t p = 0; p < PT && base + p < n_c; p++)
-                for (uint32_t b = 0; b < NB; b++) {
+                for (uint32_t b = 0; b < NB && sees(base + p); b++) {
                     const uint32_t w = s_nan[p * NB + b] >> (4u * jg);
                     nan_out |= ((uint64_t)(w & 15u) | (uint64_t)((w >> 16) & 15u) << 4) << (8u * b);
                 }
@@ -450,7 +594,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
             for (uint32_t tt = 0; tt < NT; tt++)
 #pragma unroll
                 for (uint32_t i = 0; i < 4u; i++)
-                    S[tt][i] = base + 16u * tt + 4u * jg + i < n_c ? S[tt][i] : -INFINITY;
+                    S[tt][i] = sees(base + 16u * tt + 4u * jg + i) ? S[tt][i] : -INFINITY;
         }
         float mx = -INFINITY;
 #pragma unroll
@@ -521,6 +665,17 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
                 if ((nan_out >> (4u * T + i)) & 1u) acc[T][i] = __builtin_nanf("");
     }
     const float vmul = KIND == Q4KV_Q8 ? 128.f : 1.f;
+    if constexpr (BAND) {
+        if (lo_c >= n_c) return; /* no band: written above */
+        const size_t item = (size_t)t * a.n_kvh + kh;
+        if (jg == 0u) stg((f2_t *)(a.band_ml + (item * gqa + h) * 2u), (f2_t){m_run, l});
+        float *o = a.out + ((size_t)t * a.n_head + kh * gqa + h) * HD + 4u * jg;
+#pragma unroll
+        for (uint32_t T = 0; T < TD; T++)
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; i++) stg(o + 16u * T + i, acc[T][i] * vmul);
+        return;
+    }
     if (S > 1u) {
         const uint32_t c_hi = a.n_tok * gqa - a.T1 * COLS; /* split columns per KV head */
         float *pb = a.part + (((size_t)kh * c_hi + (col - a.T1 * COLS)) * S + s) * (HD + PHEAD);
@@ -717,4 +872,32 @@ bool q4kv_dense_launch(int kind, uint32_t hd, const float *q, const void *kc, co
     else
         hd == 256u ? launch<Q4KV_F16, 256>(a) : hd == 128u ? launch<Q4KV_F16, 128>(a) : launch<Q4KV_F16, 64>(a);
     return q4kv_launch_ok("qsa dense prefill");
+}
+
+size_t q4kv_band_floats(uint32_t n_items, uint32_t gqa) { return (size_t)n_items * (1u + 2u * gqa); }
+
+bool q4kv_band_launch(AttnArgs &a, uint32_t n_items, float *part) {
+    const uint32_t gqa = a.n_head / a.n_kvh;
+    Args b = {};
+    b.kc = a.kc;
+    b.vc = a.vc;
+    b.q = a.q;
+    b.out = a.out;
+    b.n_head = a.n_head;
+    b.n_kvh = a.n_kvh;
+    b.gqa = gqa;
+    b.n_tok = n_items / a.n_kvh;
+    b.max_kv = a.max_kv;
+    b.toks = std::min(COLS / gqa, BAND_TOKS);
+    b.n_tiles = b.T1 = b.T2 = (b.n_tok + b.toks - 1u) / b.toks;
+    b.S = 1u;
+    b.scale_log2 = a.scale_log2;
+    b.idx = a.idx;
+    b.tok_stride = a.tok_stride;
+    b.kvh_stride = a.kvh_stride;
+    b.width = a.width;
+    b.band_nb = a.band_nb = (int32_t *)part;
+    b.band_ml = a.band_ml = part + n_items;
+    qsa_dense_k<Q4KV_Q8, 256, true><<<b.n_tiles * a.n_kvh, NTHR, 0, q4kv_stream>>>(b);
+    return q4kv_launch_ok("qsa band");
 }

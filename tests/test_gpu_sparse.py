@@ -1,0 +1,77 @@
+"""The listed-prefill kernel (q4kv_sparse.hip) against the oracle where it can
+go wrong: both head packings, splits and the single split with the band apart,
+lists whose length is not whole passes, padding anywhere (also whole passes
+and whole lists of it), positions past the cache, rows that are in no list and
+hold NaN, shared and per-KV-head lists."""
+import numpy as np
+import pytest
+
+import q4kv
+from gpu_util import note, quantize_on_gpu
+from synth import assert_attn_close, heads
+
+pytestmark = pytest.mark.gpu
+
+
+def _lists(rng, n, width, ctx, run):
+    """[n][width] distinct positions >= 3; some rows end in a run of `run`
+    consecutive ones (a causal window), some have padding."""
+    sel = np.empty((n, width), np.int32)
+    for t in range(n):
+        row = np.sort(rng.permutation(ctx - 3 - run)[:width]) + 3
+        if run and t % 7 != 3:
+            row[-run:] = ctx - run - (n - 1 - t) // 2 % 64 + np.arange(run)
+        sel[t] = row
+        kind = t % 5
+        if kind == 1:
+            sel[t, rng.random(width) < 0.2] = -1
+        elif kind == 2:
+            sel[t, 40:120] = -1  # whole passes
+        elif kind == 3:
+            sel[t, rng.random(width) < 0.05] = ctx + 9
+    sel[n // 2] = -1
+    return sel
+
+
+# (n_head, n_kvh, n_tok, width, per KV head, run): splits, one split, the
+# band; 9 to 16 and 1 to 8 heads per KV head
+@pytest.mark.parametrize("n_head,n_kvh,n_tok,width,per_kvh,run", [
+    (24, 2, 16, 2051, False, 0),     # 16 splits
+    (24, 2, 130, 300, False, 70),    # one split
+    (18, 2, 140, 257, True, 0),
+    (32, 2, 1030, 261, False, 90),   # the band apart, 16 heads
+    (24, 2, 1026, 256, True, 256),   # lists that are all band
+    (16, 2, 200, 259, False, 0),     # packed, 8 heads
+    (4, 2, 220, 300, True, 64),      # packed, 2 heads
+    (3, 3, 128, 290, False, 0),      # one head per KV head
+])
+def test_listed_prefill(rt, oracle, n_head, n_kvh, n_tok, width, per_kvh, run):
+    note(f"sparse heads={n_head}/{n_kvh} n_tok={n_tok} width={width} per_kvh={per_kvh} run={run}")
+    rng = np.random.default_rng(n_head * 1000 + n_tok + width)
+    ctx, hd = 2600 if width > 1000 else 1400, 256
+    k, v = heads(rng, (ctx, n_kvh)), heads(rng, (ctx, n_kvh))
+    q = heads(rng, (n_tok, n_head))
+    gate = rng.standard_normal(q.shape).astype(np.float32)
+    kc, nb = quantize_on_gpu(rt, k, q4kv.KV_Q8)
+    vc, _ = quantize_on_gpu(rt, v, q4kv.KV_Q8)
+    kb, vb = oracle.encode(k, q4kv.KV_Q8), oracle.encode(v, q4kv.KV_Q8)
+    nl = n_kvh if per_kvh else 1
+    sel = np.stack([_lists(rng, n_tok, width, ctx, run) for _ in range(nl)], 1)
+    want = oracle.attn(q, kb, vb, q4kv.KV_Q8, n_head, n_kvh, hd, n_tok, gate=gate, idx=sel.ravel(),
+                       width=width, tok_stride=nl * width, kvh_stride=width if per_kvh else 0,
+                       max_kv=ctx, threads=8)
+    for c in (kc, vc):  # rows 0-2 are in no list
+        rows = rt.download(c, nb).reshape(ctx, -1).copy()
+        rows[:3].view(np.uint16)[:, ::17] = 0x7E00
+        rt.h2d(c, rows)
+    dq, dg, di = rt.upload(q), rt.upload(gate), rt.upload(sel)
+    do = rt.alloc(q.nbytes)
+    rt.h2d(do, np.full(q.size, np.nan, np.float32))
+    assert rt.lib.q4_hip_qsa_decode_idx_kv(dq, kc, vc, dg, do, di, width, nl * width,
+                                           width if per_kvh else 0, n_head, n_kvh, hd, n_tok, ctx,
+                                           1.0 / 16, q4kv.KV_Q8)
+    rt.sync()
+    assert_attn_close(rt.download(do, q.nbytes, np.float32).reshape(q.shape), want,
+                      what=f"listed prefill gqa={n_head // n_kvh}")
+    for p in (kc, vc, dq, dg, di, do):
+        rt.free(p)
