@@ -54,6 +54,7 @@ constexpr uint32_t IDX_HD = 128;
  * address-space qualified copy, so they go through native vector types). */
 typedef float idx_f2 __attribute__((ext_vector_type(2)));
 typedef float idx_f4 __attribute__((ext_vector_type(4)));
+typedef _Float16 idx_h8 __attribute__((ext_vector_type(8)));
 __device__ inline float4 ld_vec(const float4 *p) {
     const idx_f4 v = *(const GLOBAL idx_f4 *)p;
     return make_float4(v.x, v.y, v.z, v.w);
@@ -365,138 +366,197 @@ __global__ __launch_bounds__(256) void qsa_index_score_dk(uint32_t *raw2, float 
 }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
 
-/* fp32 -> (hi, lo) bf16 pairs, both by truncation: hi = x's top 16 bits,
- * lo = the top 16 bits of x - hi (exact in fp32), so x = hi + lo to within
- * 2^-16 |x|. Two values per dword, low half first. */
-__device__ inline void split_bf16(const float4 &a, const float4 &b, s16x8 &hi, s16x8 &lo) {
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint32_t h[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t u0 = __float_as_uint(v[2 * i]), u1 = __float_as_uint(v[2 * i + 1]);
-        const uint32_t h0 = u0 & 0xffff0000u, h1 = u1 & 0xffff0000u;
-        const uint32_t l0 = __float_as_uint(v[2 * i] - __uint_as_float(h0));
-        const uint32_t l1 = __float_as_uint(v[2 * i + 1] - __uint_as_float(h1));
-        h[i] = __builtin_amdgcn_perm(h1, h0, 0x07060302u); /* {h0.hi16, h1.hi16} */
-        l[i] = __builtin_amdgcn_perm(l1, l0, 0x07060302u);
-    }
-    hi = __builtin_bit_cast(s16x8, (uint4){h[0], h[1], h[2], h[3]});
-    lo = __builtin_bit_cast(s16x8, (uint4){l[0], l[1], l[2], l[3]});
+/* Four fp32 times the power of two f -> fp16 parts, each rounded once:
+ * x f = hi + lo to 2^-22 of the row's largest magnitude. Mixed-precision fma
+ * throughout (its third operand reads fp16), two instructions per value; the
+ * two pairs alternate, so no result is read by the next instruction. */
+__device__ inline void split_h4(const float4 &x, float f, uint32_t &h0, uint32_t &h1, uint32_t &l0,
+                                uint32_t &l1) {
+    asm volatile("v_fma_mixlo_f16 %0, %4, %8, 0\n"
+                 "v_fma_mixlo_f16 %1, %6, %8, 0\n"
+                 "v_fma_mixhi_f16 %0, %5, %8, 0\n"
+                 "v_fma_mixhi_f16 %1, %7, %8, 0\n"
+                 "v_fma_mixlo_f16 %2, %4, %8, -%0 op_sel_hi:[0,0,1]\n"
+                 "v_fma_mixlo_f16 %3, %6, %8, -%1 op_sel_hi:[0,0,1]\n"
+                 "v_fma_mixhi_f16 %2, %5, %8, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n"
+                 "v_fma_mixhi_f16 %3, %7, %8, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+                 : "=&v"(h0), "=&v"(h1), "=&v"(l0), "=&v"(l1)
+                 : "v"(x.x), "v"(x.y), "v"(x.z), "v"(x.w), "v"(f));
 }
+__device__ inline void split_h8(const float4 &a, const float4 &b, float f, idx_h8 &hi, idx_h8 &lo) {
+    uint4 h, l;
+    split_h4(a, f, h.x, h.y, l.x, l.y);
+    split_h4(b, f, h.z, h.w, l.z, l.w);
+    hi = __builtin_bit_cast(idx_h8, h);
+    lo = __builtin_bit_cast(idx_h8, l);
+}
+/* max(|x|, m) over eight values; a NaN is passed over */
+__device__ inline float max_abs8(const float4 &a, const float4 &b, float m) {
+    asm("v_max3_f32 %0, |%2|, |%3|, %1" : "=v"(m) : "v"(m), "v"(a.x), "v"(a.y));
+    asm("v_max3_f32 %0, |%2|, |%3|, %1" : "=v"(m) : "v"(m), "v"(a.z), "v"(a.w));
+    asm("v_max3_f32 %0, |%2|, |%3|, %1" : "=v"(m) : "v"(m), "v"(b.x), "v"(b.y));
+    asm("v_max3_f32 %0, |%2|, |%3|, %1" : "=v"(m) : "v"(m), "v"(b.z), "v"(b.w));
+    return m;
+}
+/* the e >= lo for which |am| 2^-e is in [0.5, 1) (in [1, 4) at the top of the
+ * range: 2^-e stays normal); 0 for rows of zeros or with an infinity */
+__device__ inline int row_exp(float am, int lo) {
+    const int e = min(max(__builtin_amdgcn_frexp_expf(am), lo), 126);
+    return (am > 0.f && am <= 3.4028235e38f) ? e : 0;
+}
+/* max(x, 0), and 0 for a NaN */
+__device__ inline float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, INFINITY); }
 
-/* Block scores for a chunk of >= 4 tokens on bf16 MFMA 16x16x32 with a
- * three-product split (hi.hi + hi.lo + lo.hi, relative error ~2^-16 per
- * product, fp32 accumulation). A tile = 4 tokens x 4 heads (row 4*token +
- * head), B tile = 16 pool rows; at k-step s lane l supplies dims
- * 32s + 8(l/16) .. +7 of its row (32 contiguous bytes: a row's 128 bytes per
- * step come from its four lanes). The C layout puts one token's four heads in
- * a lane's four accumulators, so the relu-sum over heads stays in the lane.
- * Workgroup tile: 16 tokens x 256 blocks, 64 blocks per wave. */
-__global__ __launch_bounds__(256) void qsa_score_mfma_k(const float *q, const float *pool,
-                                                        float *score, uint32_t n_tok,
-                                                        uint32_t n_blocks, uint32_t stride,
-                                                        uint32_t n_head, uint32_t pos0,
-                                                        uint32_t ratio) {
-    /* the A operands (the workgroup's 16 tokens x 4 heads) are the same for
-     * its four waves: wave w loads and splits k-step w once, into LDS */
-    __shared__ s16x8 a_hi[4][4][64], a_lo[4][4][64]; /* [k-step][tile][lane] */
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i16 = lane & 15u, kq = lane >> 4;
-    const uint32_t tok0 = blockIdx.y * 16u;
-    const uint32_t blk0 = blockIdx.x * 256u + wave * 64u;
-    if (blockIdx.x * 256u >= n_blocks) return;
+/* Block scores for a chunk of >= 4 tokens on v_mfma_f32_16x16x32_f16, both
+ * operands split into two fp16 parts (hi hi + hi lo + lo hi, ~2^-21 of the
+ * rows' largest magnitudes; each row first divided by the power of two that
+ * brings its largest magnitude into [0.5, 1), and its scores multiplied back).
+ * An A tile is 4 tokens x 4 heads (row 4 token + head), so a lane's four
+ * accumulators are one token's four heads and the relu-sum stays in the lane.
+ *
+ * One workgroup: SM_TOK tokens x 32 SM_NW blocks. A wave keeps its 32 blocks' operands
+ * in registers (split once) and streams the tokens' tiles, split once per
+ * workgroup, out of LDS: 48 products per 16 LDS reads. Two B tiles interleave
+ * their blocks (column c of tile t: block 2 c + t) and neighbouring columns
+ * trade the halves of two A tiles, so a lane stores four scores; past the
+ * caches, since the rows are larger than they hold.
+ * 512 tokens x 6272 blocks: 17.5 us, of which the matrix pipe is busy for 4;
+ * the rest is the first loads and the splits (about 9) and the scores' way out.
+ * The form before it (bf16 parts by truncation, a wave of 16 tokens x 64 blocks
+ * that split its pool rows between dependent products) took 24.1, with scores
+ * 2.5e-5 from float64 where these are 1.2e-7. */
+template <uint32_t SM_TOK, uint32_t SM_NW>
+__global__ __launch_bounds__(64 * SM_NW, 4) void qsa_score_mfma_k(
+    const float *q, const float *pool, float *score, uint32_t n_tok, uint32_t n_blocks,
+    uint32_t stride, uint32_t n_head, uint32_t pos0, uint32_t ratio, int quads) {
+    constexpr uint32_t NA = SM_TOK / 4 /* A tiles */, SM_BLK = 32 * SM_NW;
+    __shared__ idx_h8 s_a[2][4][NA][64];   /* [part][k-step][tile][lane] */
+    __shared__ uint32_t s_vis[SM_TOK];
+    __shared__ __attribute__((aligned(16))) float s_qm[SM_TOK * 4]; /* 2^(e-8) of q row 4 token + head */
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t c = lane & 15u, jg = lane >> 4;
+    const uint32_t tok0 = blockIdx.y * SM_TOK, blk0 = blockIdx.x * SM_BLK + wave * 32u;
 
-    const float *ap[4];
-    bool av[4];
+    /* every load in flight together: the query tiles, eight lanes per row
+     * (8-dim units p and p + 8), and this wave's pool rows */
+    constexpr uint32_t NI = SM_TOK * 32u / (64u * SM_NW);
+    const uint32_t p8 = tid & 7u;
+    float4 x[NI][4], y[2][4][2];
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const uint32_t tok = tok0 + 4u * a + (i16 >> 2), head = i16 & 3u;
-        av[a] = tok < n_tok && head < n_head;
-        ap[a] = q + ((size_t)(av[a] ? tok : 0) * n_head + (av[a] ? head : 0)) * IDX_HD + 8u * kq;
+    for (uint32_t i = 0; i < NI; i++) {
+        const uint32_t r = (tid >> 3) + 8u * SM_NW * i, tok = tok0 + (r >> 2), head = r & 3u;
+        const bool ok = tok < n_tok && head < n_head;
+        const float *s = q + ((size_t)(ok ? tok : 0u) * n_head + (ok ? head : 0u)) * IDX_HD + 8u * p8;
+        x[i][0] = ld_vec((const float4 *)s);
+        x[i][1] = ld_vec((const float4 *)s + 1);
+        x[i][2] = ld_vec((const float4 *)(s + 64));
+        x[i][3] = ld_vec((const float4 *)(s + 64) + 1);
     }
-    const float *bp[4];
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-        uint32_t blk = blk0 + 16u * b + i16;
-        blk = blk < n_blocks ? blk : n_blocks - 1;
-        bp[b] = pool + (size_t)blk * IDX_HD + 8u * kq;
-    }
-    /* every A load is issued (ap points at a real row for any lane) and
-     * padding lanes are zeroed by a mask afterwards: a load under the lane's
-     * condition would wait for itself. The first k-step's B rows are
-     * requested in the same round trip. */
-    float4 xa[4][2], yb[2][4][2];
+    for (uint32_t t = 0; t < 2u; t++) {
+        const uint32_t blk = min(blk0 + 2u * c + t, n_blocks - 1u);
+        const float *p = pool + (size_t)blk * IDX_HD + 8u * jg;
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        xa[a][0] = ld_vec((const float4 *)(ap[a] + 32u * wave));
-        xa[a][1] = ld_vec((const float4 *)(ap[a] + 32u * wave) + 1);
-    }
-    auto load_b = [&](uint32_t st, float4 (&y)[4][2]) {
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            y[b][0] = ld_vec((const float4 *)(bp[b] + 32u * st));
-            y[b][1] = ld_vec((const float4 *)(bp[b] + 32u * st) + 1);
+        for (uint32_t st = 0; st < 4u; st++) {
+            y[t][st][0] = ld_vec((const float4 *)(p + 32u * st));
+            y[t][st][1] = ld_vec((const float4 *)(p + 32u * st) + 1);
         }
-    };
-    load_b(0u, yb[0]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const uint32_t m = av[a] ? ~0u : 0u;
-        float4 x[2];
+    for (uint32_t i = 0; i < NI; i++) {
+        const uint32_t r = (tid >> 3) + 8u * SM_NW * i; /* row 4 token + head */
+        const bool ok = tok0 + (r >> 2) < n_tok && (r & 3u) < n_head;
+        float am = max_abs8(x[i][2], x[i][3], max_abs8(x[i][0], x[i][1], 0.f));
+        am = fmaxf(am, q4kv_dpp<0xB1>(am));
+        am = fmaxf(am, q4kv_dpp<0x4E>(am));
+        am = fmaxf(am, q4kv_dpp<0x141>(am));
+        const int e = row_exp(am, -118);
+        if (p8 == 0u) s_qm[r] = ok ? __builtin_ldexpf(1.f, e - 8) : 0.f; /* - 8: no sum overflows */
+        const float f = __builtin_ldexpf(1.f, -e);
+        idx_h8 h, l;
+        /* a row's place is turned by its unit: eight lanes write eight banks' groups */
+        const uint32_t at = ((r & 15u) ^ p8) + 16u * (p8 & 3u);
+        split_h8(x[i][0], x[i][1], f, h, l);
+        s_a[0][p8 >> 2][r >> 4][at] = h;
+        s_a[1][p8 >> 2][r >> 4][at] = l;
+        split_h8(x[i][2], x[i][3], f, h, l);
+        s_a[0][2u + (p8 >> 2)][r >> 4][at] = h;
+        s_a[1][2u + (p8 >> 2)][r >> 4][at] = l;
+    }
+    if (tid < SM_TOK) s_vis[tid] = ratio ? (pos0 + tok0 + tid + 1u) / ratio : 0u;
+    idx_h8 Bh[2][4], Bl[2][4];
+    int pe[2];
 #pragma unroll
-        for (int h = 0; h < 2; h++)
-            x[h] = make_float4(__uint_as_float(__float_as_uint(xa[a][h].x) & m),
-                               __uint_as_float(__float_as_uint(xa[a][h].y) & m),
-                               __uint_as_float(__float_as_uint(xa[a][h].z) & m),
-                               __uint_as_float(__float_as_uint(xa[a][h].w) & m));
-        split_bf16(x[0], x[1], a_hi[wave][a][lane], a_lo[wave][a][lane]);
+    for (uint32_t t = 0; t < 2u; t++) {
+        float am = 0.f;
+#pragma unroll
+        for (uint32_t st = 0; st < 4u; st++) am = max_abs8(y[t][st][0], y[t][st][1], am);
+        am = fmaxf(am, __shfl_xor(am, 16));
+        am = fmaxf(am, __shfl_xor(am, 32));
+        const int e = row_exp(am, -126);
+        pe[t] = e + 8;
+        const float f = __builtin_ldexpf(1.f, -e);
+#pragma unroll
+        for (uint32_t st = 0; st < 4u; st++) split_h8(y[t][st][0], y[t][st][1], f, Bh[t][st], Bl[t][st]);
     }
     __syncthreads();
     if (blk0 >= n_blocks) return;
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
+#pragma unroll 1
+    for (uint32_t a0 = 0; a0 < NA; a0 += 2u) {
+        if (tok0 + 4u * a0 >= n_tok) break;
+        f32x4 acc[2][2];
 #pragma unroll
-    for (uint32_t st = 0; st < 4; st++) {
-        s16x8 Ah[4], Al[4], Bh[4], Bl[4];
+        for (uint32_t a = 0; a < 2u; a++)
 #pragma unroll
-        for (int a = 0; a < 4; a++) {
-            Ah[a] = a_hi[st][a][lane];
-            Al[a] = a_lo[st][a][lane];
-        }
-        if (st + 1u < 4u) load_b(st + 1u, yb[(st + 1u) & 1u]);
+            for (uint32_t t = 0; t < 2u; t++) acc[a][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int b = 0; b < 4; b++) split_bf16(yb[st & 1u][b][0], yb[st & 1u][b][1], Bh[b], Bl[b]);
+        for (uint32_t st = 0; st < 4u; st++) {
+            idx_h8 Ah[2], Al[2];
 #pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Al[a], Bh[b], acc[a][b], 0, 0, 0);
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ah[a], Bl[b], acc[a][b], 0, 0, 0);
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ah[a], Bh[b], acc[a][b], 0, 0, 0);
+            for (uint32_t a = 0; a < 2u; a++) {
+                Ah[a] = s_a[0][st][a0 + a][lane ^ (jg + 4u * (st & 1u))];
+                Al[a] = s_a[1][st][a0 + a][lane ^ (jg + 4u * (st & 1u))];
             }
-    }
-    /* lane holds C[4*kq + r][i16]: token tok0 + 4a + kq, head r, block blk0 + 16b + i16 */
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const uint32_t tok = tok0 + 4u * a + kq;
+            for (uint32_t k = 0; k < 3u; k++)
+#pragma unroll
+                for (uint32_t a = 0; a < 2u; a++)
+#pragma unroll
+                    for (uint32_t t = 0; t < 2u; t++)
+                        acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k == 0u ? Al[a] : Ah[a],
+                                                                           k == 1u ? Bl[t][st] : Bh[t][st],
+                                                                           acc[a][t], 0, 0, 0);
+        }
+        /* lane holds C[4 jg + r][c]: token tok0 + 4 a + jg, head r, blocks blk0 + 2 c, + 1 */
+        float s[2][2];
+#pragma unroll
+        for (uint32_t a = 0; a < 2u; a++) {
+            const uint32_t tl = 4u * (a0 + a) + jg, n_vis = s_vis[tl];
+            const float4 qm = *(const float4 *)(s_qm + 4u * tl);
+#pragma unroll
+            for (uint32_t t = 0; t < 2u; t++) {
+                const float v = relu(acc[a][t][0]) * qm.x + relu(acc[a][t][1]) * qm.y +
+                                relu(acc[a][t][2]) * qm.z + relu(acc[a][t][3]) * qm.w;
+                s[a][t] = blk0 + 2u * c + t < n_vis ? __builtin_ldexpf(v, pe[t]) : -1.0e30f;
+            }
+        }
+        /* even columns take tile a0's four blocks, odd ones tile a0 + 1's */
+        const bool odd = c & 1u;
+        const float g0 = odd ? s[0][0] : s[1][0], g1 = odd ? s[0][1] : s[1][1];
+        const float o0 = q4kv_dpp<0xB1>(g0), o1 = q4kv_dpp<0xB1>(g1);
+        const idx_f4 w = odd ? (idx_f4){o0, o1, s[1][0], s[1][1]} : (idx_f4){s[0][0], s[0][1], o0, o1};
+        const uint32_t tok = tok0 + 4u * (a0 + (odd ? 1u : 0u)) + jg, blk = blk0 + 2u * (c & 14u);
         if (tok >= n_tok) continue;
-        const uint32_t pos = pos0 + tok;
-        const uint32_t n_vis = ratio ? (pos + 1) / ratio : 0;
-        float *srow = score + (size_t)tok * stride;
+        float *d = score + (size_t)tok * stride + blk;
+        if (quads && blk + 3u < n_blocks) {
+            __builtin_nontemporal_store(w, (GLOBAL idx_f4 *)d);
+        } else {
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const uint32_t blk = blk0 + 16u * b + i16;
-            if (blk >= n_blocks) continue;
-            float s = 0.f;
-#pragma unroll
-            for (int r = 0; r < 4; r++) s += fmaxf(acc[a][b][r], 0.f);
-            srow[blk] = blk < n_vis ? s : -1.0e30f;
+            for (uint32_t k = 0; k < 4u; k++)
+                if (blk + k < n_blocks) stg(d + k, w[k]);
         }
     }
 }
@@ -1436,9 +1496,29 @@ extern "C" bool q4_hip_qsa_score(const float *q, const float *pool, float *score
         qsa_score_v_k<false><<<dim3(gx, n_tok), 256, 0, q4kv_stream>>>(
             q, pool, score, n_blocks, stride, n_head, pos0, ratio, nullptr);
     } else {
-        const uint32_t gx = (n_blocks + 255u) / 256u, gy = (n_tok + 15u) / 16u;
-        qsa_score_mfma_k<<<dim3(gx, gy), 256, 0, q4kv_stream>>>(q, pool, score, n_tok, n_blocks,
-                                                                stride, n_head, pos0, ratio);
+        const int quads = ((uintptr_t)score & 15u) == 0 && (stride & 3u) == 0; /* 16-byte stores */
+/* The largest workgroup that leaves the chip busy: a larger one splits each
+         * operand for more products, a smaller one has less to do before its first.
+         * Measured (us, 8 x 64 / 16 x 128 / 32 x 256 and, last, the bf16 form of
+         * 16 x 256 that these replace):
+         *   16 tokens x 6148 blocks (194 / 49 / 25 workgroups)  4.5 / 6.3 / 8.6    8.4
+         *   64 x 2016               (256 / 64 / 16)             4.2 / 5.9 / 10.2   8.3
+         *   64 x 6160               (776 / 196 / 50)            7.7 / 6.3 / 10.5   8.7
+         *   128 x 6176              (1552 / 392 / 100)          11.0 / 8.8 / 10.5  9.3
+         *   200 x 6194              (2425 / 637 / 175)          16.5 / 13.0 / 11.9 13.8
+         *   512 x 6272              (6272 / 1568 / 400)         29.6 / 20.4 / 17.5 24.1
+         *   700 x 15175             (20944 / 5236 / 1320)       95.6 / 69.1 / 50.7 59.9 */
+        const auto wgs = [&](uint32_t tok, uint32_t nw) {
+            return (uint64_t)((n_blocks + 32u * nw - 1) / (32u * nw)) * ((n_tok + tok - 1) / tok);
+        };
+        const auto go = [&](auto kernel, uint32_t tok, uint32_t nw) {
+            const dim3 grid((n_blocks + 32u * nw - 1) / (32u * nw), (n_tok + tok - 1) / tok);
+            kernel<<<grid, 64u * nw, 0, q4kv_stream>>>(q, pool, score, n_tok, n_blocks, stride,
+                                                       n_head, pos0, ratio, quads);
+        };
+        if (wgs(8, 2) <= 256u) go(qsa_score_mfma_k<8, 2>, 8, 2);
+        else if (wgs(16, 4) <= 512u) go(qsa_score_mfma_k<16, 4>, 16, 4);
+        else go(qsa_score_mfma_k<32, 8>, 32, 8);
     }
     return q4kv_launch_ok("qsa_score");
 }
