@@ -82,10 +82,9 @@ bool q4_hip_kv_append_d(void *kcache, void *vcache, const float *k, const float 
  * Value range: any finite query. The MFMA kernels divide each head's q
  * (some of them q * scale / ln 2) by the power of two that brings its
  * largest magnitude into [0.5, 1) before splitting it into fp16 parts, and
- * multiply the head's scores back (exact). The prefill band kernel (q8_0,
- * head_dim 256, prefill-sized indexed calls) dequantises K and V to fp16
- * parts like the reference's prefill tile, so cache values must stay below
- * 65504 in magnitude there. */
+ * multiply the head's scores back (exact). Cache values: whatever the width
+ * holds (the kernels that make fp16 parts of q8_0 values make them of
+ * value * scale / 128, which is in range for every finite scale). */
 /* Dense causal attention: token t of n_tok attends positions
  * 0 .. min(kv_base+t+1, max_kv)-1. q/gate/out are [n_tok][n_head][hd] fp32;
  * out = softmax(q.k*scale) @ v * sigmoid(gate) (src/q4.h:906-909). */

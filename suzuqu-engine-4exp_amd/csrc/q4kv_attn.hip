@@ -29,6 +29,10 @@
  *  - Online softmax in base 2 per chunk; the split partials (m, l, acc[hd])
  *    are merged by a second kernel that also applies the gate. A single
  *    split (prefill, or short lists) finalises in place.
+ *  - Three launches have files of their own: many tokens over one cache
+ *    (q4kv_dense.hip, also the shared window of listed prefill), decode at 64
+ *    and 128 head dims (q4kv_rows.hip) and listed prefill where one row serves
+ *    many heads (q4kv_sparse.hip). launch_kind() chooses.
  */
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
@@ -122,20 +126,9 @@ __device__ uint64_t q4kv_trace_buf[4096 * 16];
         if ((threadIdx.x & 63u) == 0 && tw_ < 4096u)                                   \
             q4kv_trace_buf[tw_ * 16u + (slot)] = wall_clock64();                       \
     } while (0)
-/* the prefill band kernel's own per-wave stamps (it runs before the slab
- * kernel of the same call, which would overwrite q4kv_trace_buf) */
-__device__ uint64_t q4kv_trace_band[4096 * 16];
-#define TRACEB(slot)                                                                   \
-    do {                                                                               \
-        const uint32_t tw_ = (blockIdx.y * gridDim.x + blockIdx.x) * (blockDim.x >> 6) + \
-                             (threadIdx.x >> 6);                                       \
-        if ((threadIdx.x & 63u) == 0 && tw_ < 4096u)                                   \
-            q4kv_trace_band[tw_ * 16u + (slot)] = wall_clock64();                      \
-    } while (0)
 #else
 #define TRACE(slot) do { } while (0)
 #define TRACEW(slot) do { } while (0)
-#define TRACEB(slot) do { } while (0)
 #endif
 
 template <int KIND> struct KCfg;
@@ -3432,11 +3425,6 @@ extern "C" bool q4_hip_qsa_step_batch_noalloc(const q4kv_step_desc *d_descs, uin
 extern "C" int q4kv_trace_read(uint64_t *host, size_t n) {
     if (hipDeviceSynchronize() != hipSuccess) return -1;
     return hipMemcpyFromSymbol(host, HIP_SYMBOL(q4kv_trace_buf), n * sizeof(uint64_t), 0,
-                               hipMemcpyDeviceToHost) == hipSuccess ? 0 : -1;
-}
-extern "C" int q4kv_trace_read_band(uint64_t *host, size_t n) {
-    if (hipDeviceSynchronize() != hipSuccess) return -1;
-    return hipMemcpyFromSymbol(host, HIP_SYMBOL(q4kv_trace_band), n * sizeof(uint64_t), 0,
                                hipMemcpyDeviceToHost) == hipSuccess ? 0 : -1;
 }
 #endif

@@ -20,10 +20,10 @@
  *   score  decode: a memory-bound stream over the pool (512 B per block);
  *          eight lanes per block row, each lane holding 16 dims of all four
  *          queries in registers, a 3-step DPP reduction per head.
- *          prefill (>= 4 tokens): bf16 MFMA 16x16x32 with a three-product
- *          hi/lo split (~2^-16 relative per product), A rows (token, head) so
- *          each lane's four accumulators are one token's four heads and the
- *          relu-sum over heads stays in the lane.
+ *          prefill (>= 4 tokens): fp16 MFMA 16x16x32 with a three-product
+ *          hi/lo split (~2^-21 relative to the rows' largest magnitudes), A
+ *          rows (token, head) so each lane's four accumulators are one token's
+ *          four heads and the relu-sum over heads stays in the lane.
  *   topk   one 1024-thread workgroup per token row, keys in VGPRs (64 per
  *          thread). One histogram pass of the distance from the row maximum
  *          (1/16-octave steps of |score|, 32-way replicated LDS counters so
