@@ -83,8 +83,11 @@ bool q4_hip_kv_append_d(void *kcache, void *vcache, const float *k, const float 
  * (some of them q * scale / ln 2) by the power of two that brings its
  * largest magnitude into [0.5, 1) before splitting it into fp16 parts, and
  * multiply the head's scores back (exact). Cache values: whatever the width
- * holds (the kernels that make fp16 parts of q8_0 values make them of
- * value * scale / 128, which is in range for every finite scale). */
+ * holds. The dense prefill, listed prefill and 64 / 128-dim decode kernels hold
+ * q8_0 V exactly, whatever its size (beside a block scale of 512 or more, so
+ * |V| up to 65000, to 2^-18). The 256-dim decode kernels and the rest of listed
+ * prefill hold weight * block scale in two fp16 parts, to 2^-25: V whose
+ * blocks stay below 0.3 lose bits there (1e-3 of the result at V x 1e-3). */
 /* Dense causal attention: token t of n_tok attends positions
  * 0 .. min(kv_base+t+1, max_kv)-1. q/gate/out are [n_tok][n_head][hd] fp32;
  * out = softmax(q.k*scale) @ v * sigmoid(gate) (src/q4.h:906-909). */

@@ -208,6 +208,32 @@ __device__ static inline uint32_t split_pk(float x, float y, float nsel) {
     return pkrtz(__builtin_fmaf(nsel, h2lo(h), x), __builtin_fmaf(nsel, h2hi(h), y));
 }
 
+/* q8_0 V as the matrix products take it: v x scale in two fp16 parts, exact
+ * for every scale below 512 (an int8 times an fp16: 19 bits, none below 2^-24;
+ * 128 x 511.75 is still fp16). Whoever meets a larger finite scale goes over to
+ * v x scale / 128 from those rows on, its accumulators with it (exact down to
+ * 2^-18, 2^-34 of the V that asks for it), and multiplies back at the end. At
+ * a fixed 1 / 128, small V lose bits: 1.5e-3 of the result at V x 1e-3, where
+ * this leaves 3e-7 as at any size. The look at every pass's scales costs 1 %
+ * (one-token decode), 0.7 % (dense prefill), 0.4 % (listed); starting over with
+ * / 128 after a loop that ended in inf - inf cost more (registers). */
+struct VScale {
+    uint32_t m = 0x3C003C00u, c = 0xE480E480u; /* 1, -1152; 1 / 128, -9 */
+    __device__ bool big() const { return m != 0x3C003C00u; }
+    __device__ void divide() {
+        m = 0x20002000u;
+        c = 0xC880C880u;
+    }
+    /* v (/ 128), exact, of x = 1024 + biased byte */
+    __device__ h2_t value(h2_t x) const {
+        return __builtin_elementwise_fma(x, __builtin_bit_cast(h2_t, m), __builtin_bit_cast(h2_t, c));
+    }
+    __device__ float undo() const { return big() ? 128.f : 1.f; }
+};
+constexpr float VSCALE_STEP = 0.0078125f;
+/* a finite fp16 of magnitude 512 or more */
+__device__ static inline bool q4kv_big_scale(uint32_t s) { return (s & 0x7C00u) - 0x6000u < 0x1C00u; }
+
 /* Decode attention at 64 and 128 head dims (q4kv_rows.hip): whether it takes
  * a shape, and its launches (mode: MODE_DENSE, MODE_INDEXED or MODE_BATCH).
  * It uses at most Q4KV_ROWS_PART floats of partials. */

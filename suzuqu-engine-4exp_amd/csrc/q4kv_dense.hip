@@ -14,9 +14,8 @@
  *    block per thread) while this pass computes, converted once for all 128
  *    columns and stored to the other LDS buffer: one barrier per pass.
  *    q8_0: K as its exact int8 values in fp16 plus the block scales in fp32,
- *    V as v * scale / 128 in two fp16 parts (the product of an int8 and an
- *    fp16 scale has at most 19 significant bits; 1 / 128 keeps the largest
- *    scale inside fp16); f16: the rows as stored;
+ *    V as v * scale in two fp16 parts, exact (VScale, one for the workgroup);
+ *    f16: the rows as stored;
  *  - S^T = K Q^T on v_mfma_f32_16x16x32_f16, Q in two fp16 parts held in
  *    registers (each column's q divided by the power of two that brings its
  *    largest magnitude into [0.5, 1)), the q8_0 block scales applied in fp32
@@ -233,6 +232,8 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     __shared__ __attribute__((aligned(16))) uint16_t s_ks[KIND == Q4KV_Q8 ? 2 : 1][KIND == Q4KV_Q8 ? NB * PT : 8];
     /* 1 + the last pass whose V rows hold a value that is not finite */
     __shared__ uint32_t s_bad[2];
+    /* 1 + the last pass with a V scale that VScale divides for */
+    __shared__ uint32_t s_big[2];
     __shared__ uint32_t s_nan[PT * NB]; /* a pass's values that are not finite, one bit each */
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -320,7 +321,8 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     const uint32_t n_pass = (n_all - lo_all + PT - 1u) / PT;
     const uint32_t p0 = (uint32_t)((uint64_t)n_pass * s / S);
     const uint32_t p1 = (uint32_t)((uint64_t)n_pass * (s + 1u) / S);
-    if (tid < 2u) s_bad[tid] = 0u;
+    if (tid < 2u) s_bad[tid] = s_big[tid] = 0u;
+    VScale vq;
 
     /* ---- this thread's share of a pass's rows ---- */
     const size_t rstride = (size_t)a.n_kvh * G::ROWB;
@@ -384,10 +386,9 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
                     u4_t wh, wl;
 #pragma unroll
                     for (uint32_t i = 0; i < 4u; i++) {
-                        /* v / 128, exact; its product with the scale rounded
-                         * once, and what the rounding left */
-                        const h2_t f = __builtin_elementwise_fma(x[i], (h2_t)((_Float16)0.0078125f),
-                                                                 (h2_t)((_Float16)-9.f));
+                        /* v, exact; its product with the scale rounded once,
+                         * and what the rounding left */
+                        const h2_t f = vq.value(x[i]);
                         const h2_t hi = f * vs;
                         wh[i] = __builtin_bit_cast(uint32_t, hi);
                         wl[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(f, vs, -hi));
@@ -397,6 +398,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
                     *(u4_t *)(s_v[buf][G::NV - 1u] + at) = wl;
                 }
                 if (masked && (sb & 0x7C00u) == 0x7C00u) s_bad[buf] = pass + 1u;
+                if (q4kv_big_scale(sb)) s_big[buf] = pass + 1u;
             }
         } else {
 #pragma unroll
@@ -477,6 +479,33 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     for (uint32_t pass = p0; pass < p1; pass++) {
         const uint32_t buf = pass & 1u, base = lo_all + pass * PT;
         const bool masked = partly(base);
+        const uint32_t big_at = KIND == Q4KV_Q8 ? s_big[buf] : 0u;
+        if (pass + 1u < p1) load(pass + 1u);
+        const uint8_t *kr = s_k[buf] + c * KS + 16u * jg;
+        const uint16_t *ksr = s_ks[KIND == Q4KV_Q8 ? buf : 0u] + 8u * jg;
+        h8_t A[8][2], ks[8];
+        auto fetch = [&](uint32_t st) {
+            const uint32_t b = st % NB, tp = st / NB;
+#pragma unroll
+            for (uint32_t k = 0; k < 2u; k++)
+                A[st][k] = *(const h8_t *)(kr + (2u * tp + k) * 16u * KS + 64u * b);
+            if constexpr (KIND == Q4KV_Q8) ks[st] = *(const h8_t *)(ksr + st * 32u);
+        };
+        fetch(0u);
+        fetch(1u);
+        if constexpr (KIND == Q4KV_Q8) {
+            /* the flag's way hides behind the operands' */
+            __builtin_amdgcn_sched_barrier(0);
+            if (!vq.big() && __builtin_amdgcn_readfirstlane(big_at) == pass + 1u) {
+                vq.divide();
+#pragma unroll
+                for (uint32_t T = 0; T < TD; T++) acc[T] *= VSCALE_STEP;
+                load(pass); /* this pass's rows once more */
+                store(pass);
+                if (pass + 1u < p1) load(pass + 1u);
+                __syncthreads();
+            }
+        }
         if (masked && s_bad[buf] == pass + 1u) {
             /* Rows that not every column sees hold inf or NaN, which a zero
              * weight would turn into NaN. They are taken out of the tile,
@@ -503,7 +532,6 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
                     nan_out |= ((uint64_t)(w & 15u) | (uint64_t)((w >> 16) & 15u) << 4) << (8u * b);
                 }
         }
-        if (pass + 1u < p1) load(pass + 1u);
         /* ---- scores: tile tt holds positions base + 16 tt + 4 jg + i of
          * column c. Eight stages of two tiles and one block; the operands of
          * the stage after next are in flight, and the scales are applied one
@@ -516,17 +544,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
             for (uint32_t tt = 0; tt < NT; tt++) Sl[tt] = (f4_t){0.f, 0.f, 0.f, 0.f};
         }
         {
-            const uint8_t *kr = s_k[buf] + c * KS + 16u * jg;
-            const uint16_t *ksr = s_ks[KIND == Q4KV_Q8 ? buf : 0u] + 8u * jg;
-            h8_t A[8][2], ks[8];
             f4_t C[8][2];
-            auto fetch = [&](uint32_t st) {
-                const uint32_t b = st % NB, tp = st / NB;
-#pragma unroll
-                for (uint32_t k = 0; k < 2u; k++)
-                    A[st][k] = *(const h8_t *)(kr + (2u * tp + k) * 16u * KS + 64u * b);
-                if constexpr (KIND == Q4KV_Q8) ks[st] = *(const h8_t *)(ksr + st * 32u);
-            };
             auto scale = [&](uint32_t st) {
                 const uint32_t tp = st / NB;
 #pragma unroll
@@ -535,8 +553,6 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
                     for (uint32_t i = 0; i < 4u; i++)
                         S[2u * tp + k][i] = fmaf((float)ks[st][4u * k + i], C[st][k][i], S[2u * tp + k][i]);
             };
-            fetch(0u);
-            fetch(1u);
 #pragma unroll
             for (uint32_t st = 0; st < 8u; st++) {
                 const uint32_t b = st % NB, tp = st / NB;
@@ -664,7 +680,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
             for (uint32_t i = 0; i < 4u; i++)
                 if ((nan_out >> (4u * T + i)) & 1u) acc[T][i] = __builtin_nanf("");
     }
-    const float vmul = KIND == Q4KV_Q8 ? 128.f : 1.f;
+    const float vmul = vq.undo();
     if constexpr (BAND) {
         if (lo_c >= n_c) return; /* no band: written above */
         const size_t item = (size_t)t * a.n_kvh + kh;

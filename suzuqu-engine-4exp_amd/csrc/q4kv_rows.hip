@@ -16,7 +16,7 @@
  *    layout (split hi / lo in the columns); lane (c, g) loads U = hd / 16
  *    consecutive dims U c .. of positions 4 g + i, and regroups them into
  *    the A operands of U tiles (tile u, row r: dim U r + u); q8_0: v x scale
- *    / 128 in two fp16 parts (exact to the last bit or two).
+ *    in two fp16 parts, exact (VScale, one for the wave).
  * An item's entries are cut into pieces of whole passes of four waves; the
  * pieces an item needs follow its own length, so a ragged batch gives every
  * workgroup the same amount of work. Items of one piece finish in place, the
@@ -121,19 +121,27 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
                 p.kw[b] = *(const GLOBAL u3u_t *)(kr + 68u * (b >> 1) + 32u * (b & 1u) + 8u * jg);
             p.ks = ldg((const uint16_t *)(kr + 34u * (jg < NB ? jg : 0u)));
         }
+        const uint8_t *vr[4];
 #pragma unroll
         for (uint32_t i = 0; i < 4u; i++) {
             const uint32_t pv = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((4u * jg + i) * 4u), (int)pk);
-            const uint8_t *vr = vbase + (size_t)pv * rstride;
+            vr[i] = vbase + (size_t)pv * rstride;
+        }
+        const uint32_t vblk = U * c / 32u;
+        if constexpr (KIND == Q4KV_Q8) { /* the scales are looked at first */
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; i++) p.vs[i] = ldg((const uint16_t *)(vr[i] + 34u * vblk));
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
             if constexpr (KIND == Q4KV_F16 && U == 8) {
-                p.v[i] = ldg((const u4_t *)(vr + 16u * c));
+                p.v[i] = ldg((const u4_t *)(vr[i] + 16u * c));
             } else if constexpr (KIND == Q4KV_F16) {
-                const u2_t x = ldg((const u2_t *)(vr + 8u * c));
+                const u2_t x = ldg((const u2_t *)(vr[i] + 8u * c));
                 p.v[i][0] = x[0];
                 p.v[i][1] = x[1];
             } else {
-                const uint32_t b = U * c / 32u;
-                const uint8_t *w = vr + 68u * (b >> 1) + 32u * (b & 1u) + (U * c & 31u);
+                const uint8_t *w = vr[i] + 68u * (vblk >> 1) + 32u * (vblk & 1u) + (U * c & 31u);
                 if constexpr (U == 8) {
                     p.vw[i] = *(const GLOBAL u3u_t *)w;
                 } else {
@@ -141,7 +149,6 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
                     p.vw[i][0] = x[0];
                     p.vw[i][1] = x[1];
                 }
-                p.vs[i] = ldg((const uint16_t *)(vr + 34u * b));
             }
         }
     };
@@ -197,6 +204,7 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) acc[k][u] = (f4_t){0.f, 0.f, 0.f, 0.f};
     }
+    VScale vq;
     const uint32_t vodd = (U * c / 32u) & 1u; /* q8_0: this lane's V block is the odd one of its pair */
 
     auto compute = [&](const Pass &p) {
@@ -234,6 +242,13 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
             }
             __builtin_amdgcn_wave_barrier();
         }
+        uint32_t vs[4], vtop = 0u;
+        if constexpr (KIND == Q4KV_Q8) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; i++) /* a stand-in row may hold inf or NaN */
+                vs[i] = (p.vmask >> (4u * jg + i)) & 1u ? p.vs[i] : 0u;
+            vtop = max(max(vs[0], vs[1]), max(vs[2], vs[3]));
+        }
         h4_t B[HG];
 #pragma unroll
         for (uint32_t k = 0; k < HG; k++) {
@@ -245,7 +260,18 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
             }
             const float mx = max32(max16(fmax2(fmax2(T[0], T[1]), fmax2(T[2], T[3]))));
             const float mn = fmax2(m_run[k], mx);
-            if (__ballot(mn > m_run[k]) != 0u) {
+            /* one branch for the maximum and for large scales (negative ones,
+             * which the quantiser never writes, and infinities come here too) */
+            if (__ballot(mn > m_run[k] || (KIND == Q4KV_Q8 && k == 0u && vtop >= 0x6000u)) != 0u) {
+                if (KIND == Q4KV_Q8 && k == 0u && !vq.big() &&
+                    __ballot(q4kv_big_scale(vs[0]) || q4kv_big_scale(vs[1]) || q4kv_big_scale(vs[2]) ||
+                             q4kv_big_scale(vs[3])) != 0u) {
+                    vq.divide();
+#pragma unroll
+                    for (uint32_t h = 0; h < HG; h++)
+#pragma unroll
+                        for (uint32_t u = 0; u < U; u++) acc[h][u] *= VSCALE_STEP;
+                }
                 const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run[k] - mn);
                 l_run[k] *= alpha;
 #pragma unroll
@@ -264,23 +290,22 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
             uint32_t x[NV][4][2];
 #pragma unroll
             for (uint32_t i = 0; i < 4u; i++) {
-                const bool ok = (p.vmask >> (4u * jg + i)) & 1u; /* a stand-in row may hold inf or NaN */
                 if constexpr (KIND == Q4KV_F16) {
+                    const bool ok = (p.vmask >> (4u * jg + i)) & 1u; /* a stand-in row may hold inf or NaN */
 #pragma unroll
                     for (uint32_t e = 0; e < 2u; e++) x[0][i][e] = ok ? p.v[i][2u * d + e] : 0u;
                 } else {
-                    const h2_t vs = (h2_t)(__builtin_bit_cast(_Float16, ok ? p.vs[i] : (uint16_t)0u));
+                    const h2_t sc = (h2_t)(__builtin_bit_cast(_Float16, (uint16_t)vs[i]));
                     const uint32_t w = __builtin_amdgcn_perm(p.vw[i][d + 1u], p.vw[i][d],
                                                              vodd ? 0x07060504u : 0x05040302u);
                     h2_t y[2];
                     biased_h4(w, y[0], y[1]);
 #pragma unroll
                     for (uint32_t e = 0; e < 2u; e++) {
-                        const h2_t f = __builtin_elementwise_fma(y[e], (h2_t)((_Float16)0.0078125f),
-                                                                 (h2_t)((_Float16)-9.f)); /* v / 128 */
-                        const h2_t hi = f * vs;
+                        const h2_t f = vq.value(y[e]);
+                        const h2_t hi = f * sc;
                         x[0][i][e] = __builtin_bit_cast(uint32_t, hi);
-                        x[NV - 1u][i][e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(f, vs, -hi));
+                        x[NV - 1u][i][e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(f, sc, -hi));
                     }
                 }
             }
@@ -308,7 +333,7 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
     }
 
     /* ---- merge the waves, then finish or leave the piece's partial ---- */
-    const float vmul = KIND == Q4KV_Q8 ? 128.f : 1.f;
+    const float vmul = vq.undo();
 #pragma unroll
     for (uint32_t k = 0; k < HG; k++) {
         const float lw = pair32_sum(sum16(l_run[k]));
@@ -320,7 +345,7 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
         for (uint32_t i = 0; i < 4u; i++) {
             float v[U];
 #pragma unroll
-            for (uint32_t u = 0; u < U; u++) v[u] = add_ror8(acc[k][u][i]);
+            for (uint32_t u = 0; u < U; u++) v[u] = add_ror8(acc[k][u][i]) * vmul;
             if (c < 8u) {
                 float *d = mrg + (wave * 8u * HG + 8u * k + c) * MROW + U * (4u * jg + i);
 #pragma unroll
@@ -342,7 +367,7 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
             v += f * *(const f4_t *)(mrg + (w * 8u * HG + g) * MROW + d);
         }
         if (np == 1u) {
-            const float inv = L > 0.f ? vmul / L : 0.f;
+            const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
             for (uint32_t i = 0; i < 4u; i++) {
                 float r = v[i] * inv;
@@ -352,7 +377,7 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
         } else {
             float *pr = a.part + (((size_t)item * ra.S + s) * gqa + g) * (HD + PHEAD);
             if (d == 0u) stg((fv2 *)pr, (fv2){M, L});
-            stg((f4_t *)(pr + PHEAD + d), v * vmul);
+            stg((f4_t *)(pr + PHEAD + d), v);
         }
     }
 }

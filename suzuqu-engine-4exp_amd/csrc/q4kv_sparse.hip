@@ -22,9 +22,9 @@
  *    columns 0-7 and 8-15 of one product, otherwise two products serve up to
  *    16 heads with one conversion of the row; the block scales are applied in
  *    fp32;
- *  - V as v x scale / 128 in two fp16 parts (exact to the last bit or two),
- *    bytes of row pairs interleaved by v_perm so that a tile's operand is 8
- *    positions of one dim: O^T += V^T P^T with no per-head scale work.
+ *  - V as v x scale in two fp16 parts, exact (VScale, one for the wave), bytes
+ *    of row pairs interleaved by v_perm so that a tile's operand is 8 positions
+ *    of one dim: O^T += V^T P^T with no per-head scale work.
  * Tile e, row 4 g + i of the output is dim 64 g + vdim(i, e).
  *
  * What bounds it: the gather (2 x 272 bytes per entry and KV head, three
@@ -43,6 +43,7 @@ namespace {
 typedef uint32_t u4u_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u2u_t __attribute__((ext_vector_type(2), aligned(4)));
 typedef float fv2 __attribute__((ext_vector_type(2)));
+typedef uint16_t us2 __attribute__((ext_vector_type(2)));
 
 constexpr uint32_t ROWB = 272, PE = 32; /* row bytes, entries per pass */
 constexpr uint32_t MROW = 260;          /* merge row: 256 dims, padded */
@@ -204,6 +205,7 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
 #pragma unroll
     for (uint32_t e = 0; e < 16u; e++) acc[e] = (f4_t){0.f, 0.f, 0.f, 0.f};
 
+    VScale vq;
     uint32_t mask_v = mask_k;
     if (q0 + wave < q1) {
         fetch(kb, kl);
@@ -331,6 +333,25 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
             }
             vs[i] = __builtin_bit_cast(h2_t, y[0] | y[1] << 16);
         }
+        /* large scales (negative ones, which the quantiser never writes, and
+         * infinities are looked at too) */
+        us2 top = __builtin_bit_cast(us2, vs[0]);
+#pragma unroll
+        for (uint32_t i = 1; i < 4u; i++) top = __builtin_elementwise_max(top, __builtin_bit_cast(us2, vs[i]));
+        if (__ballot(__builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(top, (us2)((uint16_t)0x5FFFu)))) != 0u &&
+            !vq.big()) {
+            bool b = false;
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; i++) {
+                const uint32_t y = __builtin_bit_cast(uint32_t, vs[i]);
+                b = b || q4kv_big_scale(y) || q4kv_big_scale(y >> 16);
+            }
+            if (__ballot(b) != 0u) {
+                vq.divide();
+#pragma unroll
+                for (uint32_t e = 0; e < 16u; e++) acc[e] *= VSCALE_STEP;
+            }
+        }
         /* ---- O^T += V^T P^T, four dims (one dword per row) at a time ---- */
 #pragma unroll
         for (uint32_t d = 0; d < 4u; d++) {
@@ -346,9 +367,8 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
                 u4_t ah, al;
 #pragma unroll
                 for (uint32_t r = 0; r < 4u; r++) {
-                    const h2_t f = __builtin_elementwise_fma(expand(w[r][o >> 1], o & 1u ? 0x04030402u : 0x04010400u),
-                                                             (h2_t)((_Float16)0.0078125f), (h2_t)((_Float16)-9.f));
-                    const h2_t hi = f * vs[r]; /* v / 128 x scale */
+                    const h2_t f = vq.value(expand(w[r][o >> 1], o & 1u ? 0x04030402u : 0x04010400u));
+                    const h2_t hi = f * vs[r];
                     ah[r] = __builtin_bit_cast(uint32_t, hi);
                     al[r] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(f, vs[r], -hi));
                 }
@@ -374,11 +394,12 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
         s_l[wave][lane] = lw;
     }
     float *const mrg = (float *)smem;
+    const float vmul = vq.undo();
 #pragma unroll
     for (uint32_t i = 0; i < 4u; i++)
 #pragma unroll
         for (uint32_t e = 0; e < 16u; e += 2u) {
-            fv2 v = {acc[e][i] * 128.f, acc[e + 1u][i] * 128.f};
+            fv2 v = {acc[e][i] * vmul, acc[e + 1u][i] * vmul};
             if (PACK) v = (fv2){add_ror8(v[0]), add_ror8(v[1])};
             if (c < NH) *(fv2 *)(mrg + (wave * NH + c) * MROW + 64u * jg + vdim(i, e)) = v;
         }

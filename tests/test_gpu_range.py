@@ -131,3 +131,87 @@ def test_query_magnitude_any(rt, oracle, kind, hd, n_head, n_tok, qscale):
                        n_kvh, hd, len(ts), idx=sel[ts].ravel(), width=width,
                        tok_stride=n_kvh * width, kvh_stride=width, max_kv=ctx, threads=8)
     assert_attn_close(got[ts], want, what=f"query x{qscale:g} kind {kind} hd {hd}")
+
+
+# (query heads, KV heads, head_dim, tokens, positions before them, list width:
+# 0 dense). The kernels that form fp16 parts of V: many tokens over one cache
+# (also more than 16 heads per KV head, one token and tiles split over
+# workgroups), one-token attention at 128 and 64 dims, listed prefill with 1-8
+# and 9-16 heads per KV head, and lists that are all shared window.
+V_PARTS = [(24, 2, 256, 300, 1500, 0), (32, 1, 256, 1, 1500, 0), (32, 8, 128, 300, 800, 0),
+           (16, 4, 64, 300, 800, 0), (16, 2, 128, 1, 3000, 0), (24, 2, 128, 1, 3000, 0),
+           (16, 4, 64, 1, 3000, 0), (16, 2, 256, 200, 3000, 2051), (24, 2, 256, 64, 3000, 2051),
+           (24, 2, 256, 1030, 700, 256)]
+
+
+def _v_parts(rt, oracle, case, v_of):
+    """Output of the call and the oracle's, over V = v_of(unit-scale V).
+    Queries x 0.05: scores of a few units, so that fp32 scores cost 1e-6."""
+    n_head, n_kvh, hd, n_tok, base, width = case
+    rng = np.random.default_rng(sum(case))
+    ctx = base + n_tok
+    k = heads(rng, (ctx, n_kvh), hd=hd)
+    v = v_of(heads(rng, (ctx, n_kvh), hd=hd))
+    q = heads(rng, (n_tok, n_head), hd=hd) * np.float32(0.05)
+    kc, _ = quantize_on_gpu(rt, k, 2)
+    vc, _ = quantize_on_gpu(rt, v, 2)
+    ts = np.unique(np.linspace(0, n_tok - 1, 24).astype(int))
+    kb, vb = oracle.quant_q8(k), oracle.quant_q8(v)
+    gate = np.zeros_like(q)  # sigmoid 1/2
+    if width:
+        if width == 256:
+            sel = (base + np.arange(n_tok)[:, None] - 255 + np.arange(256)).astype(np.int32)
+        else:
+            sel = np.stack([selection(rng, base + t) for t in range(n_tok)]).astype(np.int32)
+        got = gpu_idx_kv(rt, q, kc, vc, 2, n_head, n_kvh, hd, sel.ravel(), width, width, 0, ctx,
+                         gate=gate)
+    else:
+        dq, dg, do = rt.upload(q), rt.upload(gate), rt.alloc(q.nbytes)
+        assert rt.lib.q4_hip_qsa_decode_n(dq, kc, vc, dg, do, n_head, n_kvh, hd, n_tok, base, ctx,
+                                          1.0 / np.sqrt(hd), 2)
+        rt.sync()
+        got = rt.download(do, q.nbytes, np.float32).reshape(q.shape)
+        # every token's positions as a list, for the tokens that are compared
+        width = ctx
+        sel = np.tile(np.arange(ctx, dtype=np.int32), (n_tok, 1))
+        sel[sel > base + np.arange(n_tok)[:, None]] = -1
+        for p in (dq, dg, do):
+            rt.free(p)
+    for p in (kc, vc):
+        rt.free(p)
+    want = oracle.attn(q[ts], kb, vb, 2, n_head, n_kvh, hd, len(ts), gate=gate[ts],
+                       idx=sel[ts].ravel(), width=width, tok_stride=width, kvh_stride=0,
+                       max_kv=ctx, threads=8)
+    return got[ts].astype(np.float64), want.astype(np.float64)
+
+
+@pytest.mark.parametrize("case", V_PARTS)
+@pytest.mark.parametrize("vscale", [1e-1, 1e-3, 1e-5])
+def test_small_v_values(rt, oracle, case, vscale):
+    """V x 0.1 .. 1e-5 (block scales down to the fp16 subnormals): the error
+    stays relative. q, the weights and V are held to 2^-22 and the scores, a
+    few units, are fp32 sums: 4e-6 in all (2-norm; 4e-7 measured at unit
+    scale). V parts with a fixed step of 2^-18, as v * scale / 128 gives, miss
+    it from V x 0.1 on (1.6e-5, 1.5e-3 at 1e-3)."""
+    note(f"small v {case} x{vscale:g}")
+    got, want = _v_parts(rt, oracle, case, lambda v: v * np.float32(vscale))
+    assert np.linalg.norm(got - want) <= 4e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("case", V_PARTS)
+def test_v_scales_past_512(rt, oracle, case):
+    """Blocks of 32 dims scaled by 1e5 in some late rows (block scales up to
+    about 2e4, v * scale past 65504): those dims to 4e-6 of their norm, the
+    other dims to that and 2^-18, the step of v * scale / 128."""
+    note(f"v scales past 512 {case}")
+
+    def v_of(v):
+        v[v.shape[0] * 2 // 3::7, :, 32:64] *= np.float32(1e5)
+        return v
+
+    got, want = _v_parts(rt, oracle, case, v_of)
+    assert np.abs(want[..., 32:64]).max() > 400.0
+    for g, w, step in ((got[..., 32:64], want[..., 32:64], 0.0),
+                       (np.delete(got, np.s_[32:64], -1), np.delete(want, np.s_[32:64], -1),
+                        2.0 ** -18)):
+        assert np.linalg.norm(g - w) <= 4e-6 * np.linalg.norm(w) + step * np.sqrt(w.size)
