@@ -21,9 +21,9 @@
  *          eight lanes per block row, each lane holding 16 dims of all four
  *          queries in registers, a 3-step DPP reduction per head.
  *          prefill (>= 4 tokens): fp16 MFMA 16x16x32 with a three-product
- *          hi/lo split (~2^-21 relative to the rows' largest magnitudes), A
- *          rows (token, head) so each lane's four accumulators are one token's
- *          four heads and the relu-sum over heads stays in the lane.
+ *          hi/lo split (~2^-20 per product), A rows (token, head) so each
+ *          lane's four accumulators are one token's four heads and the
+ *          relu-sum over heads stays in the lane.
  *   topk   one 1024-thread workgroup per token row, keys in VGPRs (64 per
  *          thread). One histogram pass of the distance from the row maximum
  *          (1/16-octave steps of |score|, 32-way replicated LDS counters so
@@ -367,8 +367,9 @@ __global__ __launch_bounds__(256) void qsa_index_score_dk(uint32_t *raw2, float 
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-/* Four fp32 times the power of two f -> fp16 parts, each rounded once:
- * x f = hi + lo to 2^-22 of the row's largest magnitude. Mixed-precision fma
+/* Four fp32 times the power of two f -> fp16 parts, each rounded once: where
+ * f brings the row's largest magnitude into [2^14, 2^15), x f = hi + lo to
+ * 2^-22 of x or 2^-39 of that magnitude, whichever is more. Mixed-precision fma
  * throughout (its third operand reads fp16), two instructions per value; the
  * two pairs alternate, so no result is read by the next instruction. */
 __device__ inline void split_h4(const float4 &x, float f, uint32_t &h0, uint32_t &h1, uint32_t &l0,
@@ -399,19 +400,23 @@ __device__ inline float max_abs8(const float4 &a, const float4 &b, float m) {
     asm("v_max3_f32 %0, |%2|, |%3|, %1" : "=v"(m) : "v"(m), "v"(b.z), "v"(b.w));
     return m;
 }
-/* the e >= lo for which |am| 2^-e is in [0.5, 1) (in [1, 4) at the top of the
- * range: 2^-e stays normal); 0 for rows of zeros or with an infinity */
+/* the e >= lo for which |am| 2^-e is in [0.5, 1), lo keeping the powers of two
+ * formed of it in range; 0 for rows of zeros or with an infinity */
 __device__ inline int row_exp(float am, int lo) {
-    const int e = min(max(__builtin_amdgcn_frexp_expf(am), lo), 126);
+    const int e = max(__builtin_amdgcn_frexp_expf(am), lo);
     return (am > 0.f && am <= 3.4028235e38f) ? e : 0;
 }
 /* max(x, 0), and 0 for a NaN */
 __device__ inline float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, INFINITY); }
 
 /* Block scores for a chunk of >= 4 tokens on v_mfma_f32_16x16x32_f16, both
- * operands split into two fp16 parts (hi hi + hi lo + lo hi, ~2^-21 of the
- * rows' largest magnitudes; each row first divided by the power of two that
- * brings its largest magnitude into [0.5, 1), and its scores multiplied back).
+ * operands split into two fp16 parts (hi hi + hi lo + lo hi). Each row is first
+ * multiplied by the power of two that brings its largest magnitude into [2^14,
+ * 2^15), the top of fp16, and its scores are multiplied back: a product is good
+ * to 2^-20 of itself, also where q and the pool row are large in different
+ * dims, down to elements 2^-17 of their row's largest (with the largest in
+ * [0.5, 1) such rows lost bits: 1.6e-3 of the scores at 2^-14 apart, 6e-2 at
+ * 2^-20, where this leaves 1.3e-7 and 3.6e-6).
  * An A tile is 4 tokens x 4 heads (row 4 token + head), so a lane's four
  * accumulators are one token's four heads and the relu-sum stays in the lane.
  *
@@ -433,7 +438,7 @@ __global__ __launch_bounds__(64 * SM_NW, 4) void qsa_score_mfma_k(
     constexpr uint32_t NA = SM_TOK / 4 /* A tiles */, SM_BLK = 32 * SM_NW;
     __shared__ idx_h8 s_a[2][4][NA][64];   /* [part][k-step][tile][lane] */
     __shared__ uint32_t s_vis[SM_TOK];
-    __shared__ __attribute__((aligned(16))) float s_qm[SM_TOK * 4]; /* 2^(e-8) of q row 4 token + head */
+    __shared__ __attribute__((aligned(16))) float s_qm[SM_TOK * 4]; /* 2^(e-40) of q row 4 token + head */
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t c = lane & 15u, jg = lane >> 4;
     const uint32_t tok0 = blockIdx.y * SM_TOK, blk0 = blockIdx.x * SM_BLK + wave * 32u;
@@ -472,9 +477,11 @@ __global__ __launch_bounds__(64 * SM_NW, 4) void qsa_score_mfma_k(
         am = fmaxf(am, q4kv_dpp<0xB1>(am));
         am = fmaxf(am, q4kv_dpp<0x4E>(am));
         am = fmaxf(am, q4kv_dpp<0x141>(am));
-        const int e = row_exp(am, -118);
-        if (p8 == 0u) s_qm[r] = ok ? __builtin_ldexpf(1.f, e - 8) : 0.f; /* - 8: no sum overflows */
-        const float f = __builtin_ldexpf(1.f, -e);
+        const int e = row_exp(am, -109);
+        /* 2^(e-15) and, so that no sum overflows, 2^-25 that the pool row's
+         * factor gives back */
+        if (p8 == 0u) s_qm[r] = ok ? __builtin_ldexpf(1.f, e - 40) : 0.f;
+        const float f = __builtin_ldexpf(1.f, 15 - e);
         idx_h8 h, l;
         /* a row's place is turned by its unit: eight lanes write eight banks' groups */
         const uint32_t at = ((r & 15u) ^ p8) + 16u * (p8 & 3u);
@@ -495,9 +502,9 @@ __global__ __launch_bounds__(64 * SM_NW, 4) void qsa_score_mfma_k(
         for (uint32_t st = 0; st < 4u; st++) am = max_abs8(y[t][st][0], y[t][st][1], am);
         am = fmaxf(am, __shfl_xor(am, 16));
         am = fmaxf(am, __shfl_xor(am, 32));
-        const int e = row_exp(am, -126);
-        pe[t] = e + 8;
-        const float f = __builtin_ldexpf(1.f, -e);
+        const int e = row_exp(am, -112);
+        pe[t] = e + 10; /* 2^(e-15) and 2^25 */
+        const float f = __builtin_ldexpf(1.f, 15 - e);
 #pragma unroll
         for (uint32_t st = 0; st < 4u; st++) split_h8(y[t][st][0], y[t][st][1], f, Bh[t][st], Bl[t][st]);
     }
@@ -1497,7 +1504,7 @@ extern "C" bool q4_hip_qsa_score(const float *q, const float *pool, float *score
             q, pool, score, n_blocks, stride, n_head, pos0, ratio, nullptr);
     } else {
         const int quads = ((uintptr_t)score & 15u) == 0 && (stride & 3u) == 0; /* 16-byte stores */
-/* The largest workgroup that leaves the chip busy: a larger one splits each
+        /* The largest workgroup that leaves the chip busy: a larger one splits each
          * operand for more products, a smaller one has less to do before its first.
          * Measured (us, 8 x 64 / 16 x 128 / 32 x 256 and, last, the bf16 form of
          * 16 x 256 that these replace):
