@@ -55,6 +55,14 @@ __device__ inline uint32_t pieces_of(const Item &it, const RowArgs &r) {
     return p < 1u ? 1u : p < r.S ? p : r.S;
 }
 
+/* (x, y) as fp16, rounded to nearest (sel 0), or what that left (sel -1), so
+ * that both together hold 22 bits: weights cut off instead (split_pk) lower
+ * every output by 8e-8 on average */
+__device__ inline uint32_t part_pk(float x, float y, float sel) {
+    const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((fv2){x, y}, h2_t));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((fv2){fmaf(sel, h2lo(h), x), fmaf(sel, h2hi(h), y)}, h2_t));
+}
+
 /* 1024 + (byte ^ 0x80) of four bytes, in two packed fp16 pairs */
 __device__ inline void biased_h4(uint32_t w, h2_t &x, h2_t &y) {
     w ^= 0x80808080u;
@@ -190,8 +198,8 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
 #pragma unroll
         for (uint32_t b = 0; b < NB; b++)
             qB[k][b] = __builtin_bit_cast(
-                h8_t, (u4_t){split_pk(x[b][0] * qs, x[b][1] * qs, nsel), split_pk(x[b][2] * qs, x[b][3] * qs, nsel),
-                             split_pk(x[b][4] * qs, x[b][5] * qs, nsel), split_pk(x[b][6] * qs, x[b][7] * qs, nsel)});
+                h8_t, (u4_t){part_pk(x[b][0] * qs, x[b][1] * qs, nsel), part_pk(x[b][2] * qs, x[b][3] * qs, nsel),
+                             part_pk(x[b][4] * qs, x[b][5] * qs, nsel), part_pk(x[b][6] * qs, x[b][7] * qs, nsel)});
     }
     if (nq) issue(wave, e0, pa);
 
@@ -281,7 +289,7 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
 #pragma unroll
             for (uint32_t i = 0; i < 4u; i++) T[i] = __builtin_amdgcn_exp2f(T[i] - (mn == -INFINITY ? 0.f : mn));
             l_run[k] += (T[0] + T[1]) + (T[2] + T[3]);
-            B[k] = __builtin_bit_cast(h4_t, (u2_t){split_pk(T[0], T[1], nsel), split_pk(T[2], T[3], nsel)});
+            B[k] = __builtin_bit_cast(h4_t, (u2_t){part_pk(T[0], T[1], nsel), part_pk(T[2], T[3], nsel)});
         }
         /* ---- V, four dims at a time: their values at the lane's four rows
          * [part][row][dim pair], regrouped by dim ---- */

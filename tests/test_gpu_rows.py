@@ -110,3 +110,28 @@ def test_step_equals_append_then_batch(rt, oracle, kind, hd):
     assert np.array_equal(rt.download(out, q.nbytes, np.float32).reshape(q.shape), got)
     for p in [p for p in rt._owned if p not in before]:
         rt.free(p)
+
+
+@pytest.mark.parametrize("kind,n_head,n_kvh,hd", [(1, 32, 8, 128), (2, 24, 2, 128), (2, 16, 4, 64)])
+def test_weights_are_rounded(rt, oracle, kind, n_head, n_kvh, hd):
+    """Equal V everywhere, so every output is that value whatever the weights:
+    the sum of the weights' fp16 parts over the fp32 sum of the weights. Parts
+    cut off after 21 bits (an error of 0 to 2^-21, one sign) lower the mean by
+    7e-8 to 9e-8; rounded ones leave no mean but that of the fp32 sums, less
+    than the half ulp 2^-24 of a single one (1.5e-8 at most seen)."""
+    note(f"rows weights kind={kind} heads={n_head}/{n_kvh} hd={hd}")
+    rng = np.random.default_rng(3 * hd + kind)
+    n, before = 3000, set(rt._owned)
+    k, v = heads(rng, (n, n_kvh), hd=hd), np.ones((n, n_kvh, hd), np.float32)
+    q = rng.standard_normal((1, n_head, hd)).astype(np.float32) * np.float32(0.3)
+    kc, vc = rt.upload(oracle.encode(k, kind)), rt.upload(oracle.encode(v, kind))
+    value = 127.0 * float(np.float16(np.float32(1) / np.float32(127))) if kind == q4kv.KV_Q8 else 1.0
+    out = rt.alloc(q.nbytes)
+    sel = rt.upload(np.arange(n, dtype=np.int32))
+    assert rt.lib.q4_hip_qsa_decode_idx_kv(rt.upload(q), kc, vc, None, out, sel, n, n, 0, n_head,
+                                           n_kvh, hd, 1, n, 1.0 / np.sqrt(hd), kind)
+    rt.sync()
+    got = rt.download(out, q.nbytes, np.float32).astype(np.float64) / value - 1.0
+    assert abs(got.mean()) <= 2.0 ** -24, got.mean()
+    for p in [p for p in rt._owned if p not in before]:
+        rt.free(p)
