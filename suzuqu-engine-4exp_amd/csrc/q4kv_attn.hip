@@ -1794,7 +1794,7 @@ __global__ __launch_bounds__(256, 2) void qsa_slab_k(AttnArgs a) {
             const fv2 ml = ldg((const fv2 *)(a.band_ml + ((size_t)item * gqa + g) * 2u));
             mb = ml[0];
             lb = ml[1];
-            if (lb > 0.f) Mh = fmax2(Mh, mb);
+            if (lb != 0.f) Mh = fmax2(Mh, mb);
         }
         float L = 0.f;
         f4_t v = {0.f, 0.f, 0.f, 0.f};
@@ -1805,7 +1805,7 @@ __global__ __launch_bounds__(256, 2) void qsa_slab_k(AttnArgs a) {
             L += fw * s_l[w][hh];
             v += fw * *(const f4_t *)(mrg + ((w * 16u + t) * 8u + hh) * 20u + 4u * jq);
         }
-        if (lb > 0.f) {
+        if (lb != 0.f) { /* no band: 0; NaN takes part */
             const float fb = __builtin_amdgcn_exp2f(mb - Mh);
             L += fb * lb;
 #pragma unroll

@@ -722,7 +722,9 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
 }
 
 /* Merges the S partials of every split column: HD / 4 lanes per column,
- * four dims each, eight splits' rows in flight. */
+ * four dims each, eight splits' rows in flight. An empty partial has l = 0;
+ * one with l = NaN (scores that are not finite) takes part, so that a column's
+ * result does not depend on how its tile was cut. */
 template <int HD> __global__ __launch_bounds__(256) void qsa_dense_merge_k(Args a) {
     constexpr uint32_t LPC = HD / 4, CPW = 256 / LPC;
     const uint32_t c_hi = a.n_tok * a.gqa - a.T1 * COLS, kh = blockIdx.y;
@@ -748,14 +750,14 @@ template <int HD> __global__ __launch_bounds__(256) void qsa_dense_merge_k(Args 
         float mn = M;
 #pragma unroll
         for (uint32_t k = 0; k < 8u; k++)
-            if (s0 + k < a.S && ml[k][1] > 0.f) mn = max2(mn, ml[k][0]);
+            if (s0 + k < a.S && ml[k][1] != 0.f) mn = max2(mn, ml[k][0]);
         const float f = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - mn);
         L *= f;
         acc *= f;
         M = mn;
 #pragma unroll
         for (uint32_t k = 0; k < 8u; k++) {
-            if (s0 + k < a.S && ml[k][1] > 0.f) {
+            if (s0 + k < a.S && ml[k][1] != 0.f) {
                 const float w = __builtin_amdgcn_exp2f(ml[k][0] - mn);
                 L += w * ml[k][1];
                 acc += w * v[k];
@@ -764,7 +766,7 @@ template <int HD> __global__ __launch_bounds__(256) void qsa_dense_merge_k(Args 
     }
 #pragma unroll
     for (uint32_t k = 0; k < 4u; k++) {
-        const float r = L > 0.f ? acc[k] / L : 0.f;
+        const float r = L != 0.f ? acc[k] / L : 0.f;
         stg(a.out + ro + k, r * q4kv_sigmoid(g[k]));
     }
 }

@@ -392,7 +392,8 @@ __global__ __launch_bounds__(256, HG == 1 ? 3 : 2) void qsa_rows_k(RowArgs ra) {
 
 /* Merges the pieces of an (item, head) that has several: HD / 4 lanes of
  * four dims each, NG lane groups with every NG-th piece, eight of them in
- * flight per group. */
+ * flight per group. A piece without a valid entry has l = 0; one with l = NaN
+ * (scores that are not finite) takes part, as in an item of one piece. */
 template <int HD, int MODE> __global__ __launch_bounds__(256) void qsa_rows_merge_k(RowArgs ra) {
     constexpr uint32_t LPH = HD / 4, NG = 256 / LPH;
     __shared__ __attribute__((aligned(16))) f4_t s_acc[256];
@@ -423,14 +424,14 @@ template <int HD, int MODE> __global__ __launch_bounds__(256) void qsa_rows_merg
         float mn = M;
 #pragma unroll
         for (uint32_t k = 0; k < 8u; k++)
-            if (s0 + k * NG < np && ml[k][1] > 0.f) mn = fmax2(mn, ml[k][0]);
+            if (s0 + k * NG < np && ml[k][1] != 0.f) mn = fmax2(mn, ml[k][0]);
         const float f = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - mn);
         L *= f;
         acc *= f;
         M = mn;
 #pragma unroll
         for (uint32_t k = 0; k < 8u; k++)
-            if (s0 + k * NG < np && ml[k][1] > 0.f) {
+            if (s0 + k * NG < np && ml[k][1] != 0.f) {
                 const float w = __builtin_amdgcn_exp2f(ml[k][0] - mn);
                 L += w * ml[k][1];
                 acc += w * v[k];
@@ -456,7 +457,7 @@ template <int HD, int MODE> __global__ __launch_bounds__(256) void qsa_rows_merg
     }
 #pragma unroll
     for (uint32_t k = 0; k < 4u; k++) {
-        float r = L > 0.f ? acc[k] / L : 0.f;
+        float r = L != 0.f ? acc[k] / L : 0.f;
         if (it.gate) r *= q4kv_sigmoid(gt[k]);
         stg(it.out + (size_t)g * HD + d + k, r);
     }

@@ -409,11 +409,11 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
         float M = -INFINITY, mb = -INFINITY, lb = 0.f;
 #pragma unroll
         for (uint32_t w = 0; w < 4u; w++) M = fmax2(M, s_m[w][g]);
-        if (band) { /* the band's partial, its rows in out */
+        if (band) { /* the band's partial, its rows in out (none: l = 0; l may be NaN) */
             const fv2 ml = ldg((const fv2 *)(a.band_ml + ((size_t)item * gqa + g) * 2u));
             mb = ml[0];
             lb = ml[1];
-            if (lb > 0.f) M = fmax2(M, mb);
+            if (lb != 0.f) M = fmax2(M, mb);
         }
         float L = 0.f;
         f4_t v = {0.f, 0.f, 0.f, 0.f};
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
             v += f * *(const f4_t *)(mrg + (w * NH + g) * MROW + d);
         }
         float *const o = it.out + (size_t)g * 256u + d;
-        if (lb > 0.f) {
+        if (lb != 0.f) {
             const float f = __builtin_amdgcn_exp2f(mb - M);
             L += f * lb;
 #pragma unroll

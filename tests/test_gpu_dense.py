@@ -96,3 +96,42 @@ def test_values_not_finite(rt, kind, hd):
     assert np.array_equal(got[~hit], clean[~hit])
     for p in (kc, vc):
         rt.free(p)
+
+
+@pytest.mark.parametrize("kind,hd", [(2, 256), (1, 256), (2, 128), (1, 64)])
+def test_scores_not_finite(rt, kind, hd):
+    """A NaN in one head's query: that head's row of that token is NaN, whether
+    its tile is split or not, and no other one. A NaN in a K row: every token
+    that sees the row is NaN in that KV head, no other one. (The others may
+    round differently: a wave's columns move their maxima together.)"""
+    n_head, n_kvh = 24, 2
+    # the last half of the tiles is split (64 dims: all)
+    n_tok, base = {256: (700, 0), 128: (1000, 0), 64: (300, 3000)}[hd]
+    ctx = base + n_tok
+    note(f"dense scores not finite kind={kind} hd={hd}")
+    k, v, q, gate = _inputs(7 + hd, kind, n_head, n_kvh, hd, n_tok, ctx)
+    kc, nb = quantize_on_gpu(rt, k, kind)
+    vc, _ = quantize_on_gpu(rt, v, kind)
+    clean = _run(rt, q, gate, kc, vc, kind, n_kvh, base, ctx)
+    assert np.isfinite(clean).all()
+    hit = np.zeros(q.shape, bool)
+    qn = q.copy()
+    for t in (0, 9, n_tok // 2, n_tok - 50, n_tok - 1):
+        qn[t, (t * 5) % n_head, t % hd] = np.nan
+        hit[t, (t * 5) % n_head] = True
+    got = _run(rt, qn, gate, kc, vc, kind, n_kvh, base, ctx)
+    assert np.isnan(got[hit]).all()
+    assert_attn_close(got[~hit], clean[~hit])
+    for row, kh in ((base + 40, 1), (ctx - 60, 0)):
+        rows = rt.download(kc, nb).reshape(ctx, n_kvh, -1)
+        bad = rows.copy()
+        bad[row, kh].view(np.uint16)[17 if kind == q4kv.KV_Q8 else 40] = 0x7E00
+        rt.h2d(kc, bad)
+        got = _run(rt, q, gate, kc, vc, kind, n_kvh, base, ctx)
+        rt.h2d(kc, rows)
+        hit = np.zeros(q.shape, bool)
+        hit[row - base:, kh * 12:kh * 12 + 12] = True
+        assert np.isnan(got[hit]).all()
+        assert_attn_close(got[~hit], clean[~hit])
+    for p in (kc, vc):
+        rt.free(p)

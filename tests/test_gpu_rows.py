@@ -135,3 +135,30 @@ def test_weights_are_rounded(rt, oracle, kind, n_head, n_kvh, hd):
     assert abs(got.mean()) <= 2.0 ** -24, got.mean()
     for p in [p for p in rt._owned if p not in before]:
         rt.free(p)
+
+
+@pytest.mark.parametrize("kind,hd", [(1, 128), (2, 64)])
+def test_scores_not_finite(rt, oracle, kind, hd):
+    """A NaN in a head's query, or in a K row, reaches that head's (that KV
+    head's) output whether the item is one piece or many."""
+    note(f"rows scores not finite kind={kind} hd={hd}")
+    rng = np.random.default_rng(hd)
+    n_head, n_kvh, before = 16, 4, set(rt._owned)
+    out = rt.alloc(n_head * hd * 4)
+    for n in (60, 5000):
+        k, v = heads(rng, (n, n_kvh), hd=hd), heads(rng, (n, n_kvh), hd=hd)
+        q = heads(rng, (1, n_head), hd=hd)
+        gate = rt.upload(np.zeros_like(q))
+        kb, vc = oracle.encode(k, kind), rt.upload(oracle.encode(v, kind))
+        qn, kn = q.copy(), kb.copy()
+        qn[0, 5, 7] = np.nan
+        kn.view(np.uint8).reshape(n, n_kvh, -1)[n // 3, 2].view(np.uint16)[17] = 0x7E00
+        for qx, kx, hit in ((qn, kb, [5]), (q, kn, [8, 9, 10, 11])):
+            assert rt.lib.q4_hip_qsa_decode(rt.upload(qx), rt.upload(kx), vc, gate, out, n_head,
+                                            n_kvh, hd, n, n, 1.0 / np.sqrt(hd), kind)
+            rt.sync()
+            got = rt.download(out, q.nbytes, np.float32).reshape(n_head, hd)
+            assert np.isnan(got[hit]).all(), n
+            assert np.isfinite(np.delete(got, hit, 0)).all(), n
+    for p in [p for p in rt._owned if p not in before]:
+        rt.free(p)

@@ -75,3 +75,39 @@ def test_listed_prefill(rt, oracle, n_head, n_kvh, n_tok, width, per_kvh, run):
                       what=f"listed prefill gqa={n_head // n_kvh}")
     for p in (kc, vc, dq, dg, di, do):
         rt.free(p)
+
+
+@pytest.mark.parametrize("n_head,n_tok", [(24, 1030), (16, 1030)])
+def test_scores_not_finite(rt, n_head, n_tok):
+    """A NaN in a K row reaches the tokens that list it, in the shared window
+    (attended apart) as well as before it; both kernels that take the rest."""
+    note(f"sparse scores not finite heads={n_head} n_tok={n_tok}")
+    n_kvh, hd, width, run = 2, 256, 261, 90
+    rng = np.random.default_rng(n_head)
+    ctx = 1400
+    sel = _lists(rng, n_tok, width, ctx, run)
+    q = heads(rng, (n_tok, n_head))
+    k, v = heads(rng, (ctx, n_kvh)), heads(rng, (ctx, n_kvh))
+    kc, nb = quantize_on_gpu(rt, k, q4kv.KV_Q8)
+    vc, _ = quantize_on_gpu(rt, v, q4kv.KV_Q8)
+    dq, di, do = rt.upload(q), rt.upload(sel), rt.alloc(q.nbytes)
+
+    def run_once():
+        assert rt.lib.q4_hip_qsa_decode_idx_kv(dq, kc, vc, None, do, di, width, width, 0, n_head,
+                                               n_kvh, hd, n_tok, ctx, 1.0 / 16, q4kv.KV_Q8)
+        rt.sync()
+        return rt.download(do, q.nbytes, np.float32).reshape(q.shape)
+
+    assert np.isfinite(run_once()).all()
+    rows = rt.download(kc, nb).reshape(ctx, n_kvh, -1)
+    for row in (ctx - 70, 100):  # a window row, a row before the windows
+        bad = rows.copy()
+        bad[row, 1].view(np.uint16)[17] = 0x7E00
+        rt.h2d(kc, bad)
+        got = run_once()
+        hit = np.zeros(q.shape, bool)
+        hit[(sel == row).any(1), n_head // 2:] = True
+        assert hit.any() and np.isnan(got[hit]).all()
+        assert np.isfinite(got[~hit]).all()
+    for p in (kc, vc, dq, di, do):
+        rt.free(p)
