@@ -153,11 +153,34 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
                 dma16(base + (uint64_t)p * rstride + ((x >> 7) & 0x1FFu), dst + u * 1024u);
         }
     };
+    /* The first of this wave's passes q, q + 4, .. that has a valid entry (q1
+     * or more: none), eight passes a round trip: a short context's list is
+     * padded to the width, and no rows are fetched for that. */
+    auto seek = [&](uint32_t q) {
+        for (; q < q1; q += 32u) {
+            int32_t e[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; k++) e[k] = entry(q + 8u * k + (lane >> 5) * 4u);
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; k++) {
+                const uint32_t p = q + 8u * k;
+                const uint64_t b = __ballot(PE * (p + (lane >> 5) * 4u) + (lane & 31u) < n && e[k] >= 0 &&
+                                            (uint32_t)e[k] < it.max_kv);
+                if ((uint32_t)b) return p;
+                if (b) return p + 4u;
+            }
+        }
+        return q1;
+    };
     int32_t e0 = 0;
-    if (q0 + wave < q1) {
-        e0 = entry(q0 + wave);
-        place(q0 + wave, e0);
-        e0 = entry(q0 + wave + 4u);
+    uint32_t q = q0 + wave;
+    if (q < q1) {
+        place(q, entry(q));
+        if (!mask_k) {
+            q = seek(q + 4u);
+            if (q < q1) place(q, entry(q));
+        }
+        if (q < q1) e0 = entry(q + 4u);
     }
 
     /* ---- Q^T operands in registers: column c, k-group jg ---- */
@@ -207,11 +230,11 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
 
     VScale vq;
     uint32_t mask_v = mask_k;
-    if (q0 + wave < q1) {
+    if (q < q1) {
         fetch(kb, kl);
         fetch(vb, vl);
     }
-    for (uint32_t q = q0 + wave; q < q1; q += 4u) {
+    while (q < q1) {
         /* ---- scores, once the K rows have landed (nine V instructions and
          * the list entry may be out) ---- */
         asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
@@ -276,7 +299,12 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
          * also covers the V rows */
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         mask_v = mask_k;
-        place(q + 4u, e0);
+        q += 4u;
+        place(q, e0);
+        if (!mask_k && q < q1) {
+            q = seek(q + 4u);
+            if (q < q1) place(q, entry(q));
+        }
         fetch(kb, kl);
         /* ---- softmax (base 2) over the entries of mask_v ---- */
         const uint32_t mask_l = mask_v >> (4u * jg); /* the lane's: bits 0-3 and 16-19 */
@@ -381,7 +409,7 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* V reads returned: refill */
-        e0 = entry(q + 8u);
+        e0 = entry(q + 4u);
         fetch(vb, vl);
     }
 

@@ -111,3 +111,40 @@ def test_scores_not_finite(rt, n_head, n_tok):
         assert np.isfinite(got[~hit]).all()
     for p in (kc, vc, dq, di, do):
         rt.free(p)
+
+
+@pytest.mark.parametrize("n_head,n_tok,width", [(24, 40, 2051), (24, 260, 2051), (16, 210, 2051),
+                                                (24, 1030, 700)])
+def test_mostly_padding(rt, oracle, n_head, n_tok, width):
+    """Lists of a prompt's first tokens (t + 1 positions, then padding) and
+    lists with a few entries in passes far apart: passes without an entry are
+    passed over, at the start, in between and at the end of a wave's share."""
+    note(f"sparse padding heads={n_head} n_tok={n_tok} width={width}")
+    n_kvh, hd, ctx = 2, 256, 1400
+    rng = np.random.default_rng(n_head + n_tok)
+    sel = np.full((n_tok, width), -1, np.int32)
+    for t in range(n_tok):
+        if t % 3 == 2:  # 1 to 12 entries anywhere
+            at = rng.choice(width, 1 + t % 12, replace=False)
+            sel[t, at] = rng.choice(ctx, at.size, replace=False)
+        elif t % 3 == 1:  # one entry alone: the list's first, last, any pass
+            sel[t, (0, width - 1, 32 * (t % (width // 32)))[t // 3 % 3]] = t
+        else:
+            n = min(t + 1, width, ctx)
+            sel[t, :n] = np.arange(n)
+    k, v = heads(rng, (ctx, n_kvh)), heads(rng, (ctx, n_kvh))
+    q = heads(rng, (n_tok, n_head))
+    kc, _ = quantize_on_gpu(rt, k, q4kv.KV_Q8)
+    vc, _ = quantize_on_gpu(rt, v, q4kv.KV_Q8)
+    want = oracle.attn(q, oracle.encode(k, 2), oracle.encode(v, 2), q4kv.KV_Q8, n_head, n_kvh, hd,
+                       n_tok, idx=sel.ravel(), width=width, tok_stride=width, kvh_stride=0,
+                       max_kv=ctx, threads=8)
+    dq, di, do = rt.upload(q), rt.upload(sel), rt.alloc(q.nbytes)
+    rt.h2d(do, np.full(q.size, np.nan, np.float32))
+    assert rt.lib.q4_hip_qsa_decode_idx_kv(dq, kc, vc, None, do, di, width, width, 0, n_head,
+                                           n_kvh, hd, n_tok, ctx, 1.0 / 16, q4kv.KV_Q8)
+    rt.sync()
+    assert_attn_close(rt.download(do, q.nbytes, np.float32).reshape(q.shape), want,
+                      what=f"padding gqa={n_head // n_kvh}")
+    for p in (kc, vc, dq, di, do):
+        rt.free(p)
