@@ -3020,9 +3020,11 @@ static bool launch_sparse(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t
     a.item0 = 0u;
     a.band_nb = nullptr;
     a.band_ml = nullptr;
-    /* the shared window apart: 1024 tokens, 24 / 2 heads: 329 against 344 us;
-     * 512: 198 against 180 */
-    if (S == 1u && n_items >= 2048u && band_enabled() && pb.ptr && q4kv_band_floats(n_items, gqa) <= pb.cap) {
+    /* The shared window apart, where it is part of a long list: 24 / 2 heads,
+     * 1024 tokens, with and without it: 338 / 345 us at 2051 entries, 272 / 273
+     * at 1536, 210 / 209 at 1024, 148 / 138 at 512 (a quarter of them window);
+     * 512 tokens at 2051: 198 / 180. */
+    if (S == 1u && n_items >= 2048u && max_n > 1536u && band_enabled() && pb.ptr && q4kv_band_floats(n_items, gqa) <= pb.cap) {
         if (!q4kv_band_launch(a, n_items, pb.ptr)) return false;
     }
     if (!q4kv_sparse_launch(a, n_items)) return false;

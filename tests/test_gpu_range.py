@@ -141,7 +141,7 @@ def test_query_magnitude_any(rt, oracle, kind, hd, n_head, n_tok, qscale):
 V_PARTS = [(24, 2, 256, 300, 1500, 0), (32, 1, 256, 1, 1500, 0), (32, 8, 128, 300, 800, 0),
            (16, 4, 64, 300, 800, 0), (16, 2, 128, 1, 3000, 0), (24, 2, 128, 1, 3000, 0),
            (16, 4, 64, 1, 3000, 0), (16, 2, 256, 200, 3000, 2051), (24, 2, 256, 64, 3000, 2051),
-           (24, 2, 256, 1030, 700, 256)]
+           (16, 2, 256, 1030, 700, 256)]
 
 
 def _v_parts(rt, oracle, case, v_of):

@@ -39,8 +39,10 @@ def _lists(rng, n, width, ctx, run):
     (24, 2, 16, 2051, False, 0),     # 16 splits
     (24, 2, 130, 300, False, 70),    # one split
     (18, 2, 140, 257, True, 0),
-    (32, 2, 1030, 261, False, 90),   # the band apart, 16 heads
+    (32, 2, 1030, 261, False, 90),   # many tokens, short lists: the band stays in them
     (24, 2, 1026, 256, True, 256),   # lists that are all band
+    (32, 2, 1030, 1537, False, 500), # the band apart, 16 heads
+    (18, 2, 1025, 1600, True, 90),
     (16, 2, 200, 259, False, 0),     # packed, 8 heads
     (4, 2, 220, 300, True, 64),      # packed, 2 heads
     (3, 3, 128, 290, False, 0),      # one head per KV head
@@ -77,14 +79,14 @@ def test_listed_prefill(rt, oracle, n_head, n_kvh, n_tok, width, per_kvh, run):
         rt.free(p)
 
 
-@pytest.mark.parametrize("n_head,n_tok", [(24, 1030), (16, 1030)])
-def test_scores_not_finite(rt, n_head, n_tok):
+@pytest.mark.parametrize("n_head,n_tok,width", [(24, 1030, 1537), (16, 1030, 261)])
+def test_scores_not_finite(rt, n_head, n_tok, width):
     """A NaN in a K row reaches the tokens that list it, in the shared window
     (attended apart) as well as before it; both kernels that take the rest."""
     note(f"sparse scores not finite heads={n_head} n_tok={n_tok}")
-    n_kvh, hd, width, run = 2, 256, 261, 90
+    n_kvh, hd, run = 2, 256, 90
     rng = np.random.default_rng(n_head)
-    ctx = 1400
+    ctx = 2600 if width > 1000 else 1400
     sel = _lists(rng, n_tok, width, ctx, run)
     q = heads(rng, (n_tok, n_head))
     k, v = heads(rng, (ctx, n_kvh)), heads(rng, (ctx, n_kvh))
