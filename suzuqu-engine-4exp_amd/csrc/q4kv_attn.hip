@@ -2832,7 +2832,15 @@ struct Plan {
  * Q4KV_SLAB=0 turns the slab kernel off, Q4KV_SLAB=2 uses it everywhere
  * (A/B measurement). */
 #define SLAB_MAX_WG 16384u
-#define SLAB_SPLIT_WG 1024u /* workgroups a prefill-sized launch is split to */
+/* Workgroups a prefill-sized launch is split to. Listed tokens are alike, so
+ * about one round of workgroups is enough (512 tokens x 4 KV heads: 291 us,
+ * 352 with 16384). A batch's items are as long as they like, and pieces of the
+ * long ones have to fill in behind the short. Dense items, 1024 / 3072 / 16384
+ * workgroups: 48 sequences of 1000 to 60000 positions, 16 / 2 heads 219 / 192 /
+ * 204 us, 24 / 2 heads 428 / 291 / 291, 8 / 8 heads 433 / 282 / 405; 96 of 500
+ * to 40000, 24 / 2 heads 541 / 406 / 407; 48 of 24000, 16 / 2 heads 240 / 257 /
+ * 270, 24 / 2 heads 382 / 408 / 408. */
+#define SLAB_SPLIT_WG(mode) (IS_BATCH(mode) ? 3072u : 1024u)
 static int slab_mode(void) {
     static int v = -1;
     if (v < 0) {
@@ -2931,7 +2939,7 @@ static Plan plan_launch(uint32_t hd, uint32_t n_items, uint32_t max_n, uint32_t 
         if (!prefill_sized) {
             choose_split(n_items, s_full, gqa, have_part, cap, S, cps);
         } else {
-            S = n_items >= SLAB_SPLIT_WG ? 1u : SLAB_SPLIT_WG / n_items;
+            S = n_items >= SLAB_SPLIT_WG(MODE) ? 1u : SLAB_SPLIT_WG(MODE) / n_items;
             if (S < 1u) S = 1u;
             if (S > COMB_REG) S = COMB_REG; /* the merge's register path */
             const size_t per = (size_t)gqa * PSTRIDE;
