@@ -787,7 +787,7 @@ template <int KIND, int HD> void launch(const Args &a) {
  * the tiles are alike; a workgroup's start and end (START); the
  * merge launch (MERGE) and the partials, 128 KB written and read per piece
  * (PART). */
-constexpr uint32_t N_CU = 256;
+constexpr uint32_t N_CU = 256, MAX_SPLIT = 64;
 constexpr float START = 4.f, MERGE = 3.f, PART = 0.04f;
 
 void plan(Args &a, uint32_t hd, size_t cap) {
@@ -804,7 +804,7 @@ void plan(Args &a, uint32_t hd, size_t cap) {
     if (!a.part || a.n_kvh > 65535u) return;
     float best = 1e30f;
     const float spread = (n_hi - n_lo) / n_hi;
-    static const uint32_t cand[] = {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, 24u, 32u, 48u, 64u};
+    static const uint32_t cand[] = {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, 24u, 32u, 48u, MAX_SPLIT};
     for (uint32_t S : cand) {
         if (S > 1u && 2u * S > (uint32_t)n_hi) break;
         for (uint32_t k = 0; k < 4u; k++) { /* split the last 4 - k quarters of the tiles */
@@ -858,11 +858,29 @@ bool q4kv_dense_takes(int kind, uint32_t hd, uint32_t n_tok, uint32_t n_kvh, uin
      * tokens: 27.6 against 23.8 over 1000, 37.3 against 46.7 over 4000.
      * 64 and 128 dims (q4kv_rows.hip), 160 thousand: 32 / 8 heads of 128
      * dims: 13.6 against 12.1 us for 8 tokens over 1000 positions, 30.7
-     * against 32.1 for 2 over 16000, 32.0 against 86.9 for 8. */
+     * against 32.1 for 2 over 16000, 32.0 against 86.9 for 8.
+     * And where a column tile stands for enough of those slots: a few tokens
+     * leave most of its 128 columns empty, and one tile of a long cache is cut
+     * into MAX_SPLIT pieces at most. 8 heads per KV head, us by tokens, this
+     * kernel against the others: q8_0, 2 KV heads, 130 thousand positions: 2:
+     * 165 / 65, 4: 167 / 84, 8: 170 / 149, 16: 173 / 299; 40 thousand: 4: 66 /
+     * 48, 8: 69 / 55; 8 KV heads of 4, 40 thousand: 2: 106 / 55, 4: 107 / 93, 6:
+     * 108 / 116; f16, 2 KV heads, 130 thousand: 2: 116 / 76, 3: 117 / 99, 6: 119 /
+     * 169; q8_0 of 128 dims, 130 thousand: 2: 95 / 64, 4: 96 / 89, 6: 97 / 119. */
     if (gqa > 16u) return true;
-    const uint64_t slots = (uint64_t)n_tok * n_kvh * (gqa > 8u ? 2u : 1u) *
-                           (max_n - std::min<uint64_t>(max_n, n_tok) / 2u);
-    return n_tok > 1u && slots > (hd == 256u ? 280000u : 160000u);
+    if (n_tok < 2u) return false;
+    const uint32_t hg = gqa > 8u ? 2u : 1u;
+    const uint64_t slots = (uint64_t)n_tok * n_kvh * hg * (max_n - std::min<uint64_t>(max_n, n_tok) / 2u);
+    const float tiles = (float)((cols + COLS - 1u) / COLS) * n_kvh; /* and the CUs that they fill */
+    const float per_tile = (float)n_tok * n_kvh * hg / tiles * std::min(1.f, tiles * MAX_SPLIT / N_CU);
+    if (slots <= (hd == 256u ? 280000u : 160000u)) return false;
+    if (kind == Q4KV_F16 || hd == 64u) return per_tile > 1.5f;
+    if (hd == 128u) return per_tile > 2.f;
+    /* the others fall back past a size: 6 tokens, 2 KV heads, 130 thousand
+     * positions: 163 / 222; 3 tokens, 8 KV heads, 60 thousand: 146 / 173 (40
+     * thousand: 105 / 78); 12 heads per KV head, 3 tokens: 40 thousand 66 / 60,
+     * 60 thousand 87 / 117 */
+    return per_tile > (gqa > 8u ? 3.f : 4.f) || (per_tile > 2.5f && slots > (gqa > 8u ? 600000u : 1300000u));
 }
 
 bool q4kv_dense_launch(int kind, uint32_t hd, const float *q, const void *kc, const void *vc,
