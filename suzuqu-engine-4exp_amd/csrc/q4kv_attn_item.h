@@ -215,8 +215,9 @@ __device__ static inline uint32_t split_pk(float x, float y, float nsel) {
  * 2^-18, 2^-34 of the V that asks for it), and multiplies back at the end. At
  * a fixed 1 / 128, small V lose bits: 1.5e-3 of the result at V x 1e-3, where
  * this leaves 3e-7 as at any size. The look at every pass's scales costs 1 %
- * (one-token decode), 0.7 % (dense prefill), 0.4 % (listed); starting over with
- * / 128 after a loop that ended in inf - inf cost more (registers). */
+ * (one-token decode, listed prefill) or less (dense prefill), in the branch of
+ * the running maximum where there is room; starting over with / 128 after a
+ * loop that ended in inf - inf cost more (registers). */
 struct VScale {
     uint32_t m = 0x3C003C00u, c = 0xE480E480u; /* 1, -1152; 1 / 128, -9 */
     __device__ bool big() const { return m != 0x3C003C00u; }

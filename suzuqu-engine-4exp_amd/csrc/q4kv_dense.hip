@@ -230,10 +230,10 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     /* K block scales, in the order the score stages read them: [tile pair]
      * [block][k-group][tile][position], 16 bytes per lane and stage */
     __shared__ __attribute__((aligned(16))) uint16_t s_ks[KIND == Q4KV_Q8 ? 2 : 1][KIND == Q4KV_Q8 ? NB * PT : 8];
-    /* 1 + the last pass whose V rows hold a value that is not finite */
-    __shared__ uint32_t s_bad[2];
-    /* 1 + the last pass with a V scale that VScale divides for */
-    __shared__ uint32_t s_big[2];
+    /* 1 + the last pass whose V rows hold a value that is not finite; 1 + the
+     * last one with a V scale that VScale divides for (mod 2^16: what either
+     * leads to is right, if not needed, at any pass) */
+    __shared__ __attribute__((aligned(4))) uint16_t s_flag[2][2];
     __shared__ uint32_t s_nan[PT * NB]; /* a pass's values that are not finite, one bit each */
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
     const uint32_t n_pass = (n_all - lo_all + PT - 1u) / PT;
     const uint32_t p0 = (uint32_t)((uint64_t)n_pass * s / S);
     const uint32_t p1 = (uint32_t)((uint64_t)n_pass * (s + 1u) / S);
-    if (tid < 2u) s_bad[tid] = s_big[tid] = 0u;
+    if (tid < 4u) s_flag[tid >> 1][tid & 1u] = 0u;
     VScale vq;
 
     /* ---- this thread's share of a pass's rows ---- */
@@ -397,8 +397,8 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
                     *(u4_t *)(s_v[buf][0] + at) = wh;
                     *(u4_t *)(s_v[buf][G::NV - 1u] + at) = wl;
                 }
-                if (masked && (sb & 0x7C00u) == 0x7C00u) s_bad[buf] = pass + 1u;
-                if (q4kv_big_scale(sb)) s_big[buf] = pass + 1u;
+                if (masked && (sb & 0x7C00u) == 0x7C00u) s_flag[buf][0] = (uint16_t)(pass + 1u);
+                if (q4kv_big_scale(sb)) s_flag[buf][1] = (uint16_t)(pass + 1u);
             }
         } else {
 #pragma unroll
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
                     for (uint32_t k = 0; k < 4u; k++)
                         bad = bad || (rv[i][k] & 0x7C00u) == 0x7C00u ||
                               (rv[i][k] & 0x7C000000u) == 0x7C000000u;
-                    if (bad) s_bad[buf] = pass + 1u;
+                    if (bad) s_flag[buf][0] = (uint16_t)(pass + 1u);
                 }
             }
         }
@@ -472,66 +472,15 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
 #pragma unroll
     for (uint32_t T = 0; T < TD; T++) acc[T] = (f4_t){0.f, 0.f, 0.f, 0.f};
 
-    __syncthreads(); /* s_bad cleared */
+    __syncthreads(); /* s_flag cleared */
     if (p0 < p1) store(p0);
     __syncthreads();
 
     for (uint32_t pass = p0; pass < p1; pass++) {
         const uint32_t buf = pass & 1u, base = lo_all + pass * PT;
         const bool masked = partly(base);
-        const uint32_t big_at = KIND == Q4KV_Q8 ? s_big[buf] : 0u;
+        const uint32_t flag_at = *(const uint32_t *)s_flag[buf];
         if (pass + 1u < p1) load(pass + 1u);
-        const uint8_t *kr = s_k[buf] + c * KS + 16u * jg;
-        const uint16_t *ksr = s_ks[KIND == Q4KV_Q8 ? buf : 0u] + 8u * jg;
-        h8_t A[8][2], ks[8];
-        auto fetch = [&](uint32_t st) {
-            const uint32_t b = st % NB, tp = st / NB;
-#pragma unroll
-            for (uint32_t k = 0; k < 2u; k++)
-                A[st][k] = *(const h8_t *)(kr + (2u * tp + k) * 16u * KS + 64u * b);
-            if constexpr (KIND == Q4KV_Q8) ks[st] = *(const h8_t *)(ksr + st * 32u);
-        };
-        fetch(0u);
-        fetch(1u);
-        if constexpr (KIND == Q4KV_Q8) {
-            /* the flag's way hides behind the operands' */
-            __builtin_amdgcn_sched_barrier(0);
-            if (!vq.big() && __builtin_amdgcn_readfirstlane(big_at) == pass + 1u) {
-                vq.divide();
-#pragma unroll
-                for (uint32_t T = 0; T < TD; T++) acc[T] *= VSCALE_STEP;
-                load(pass); /* this pass's rows once more */
-                store(pass);
-                if (pass + 1u < p1) load(pass + 1u);
-                __syncthreads();
-            }
-        }
-        if (masked && s_bad[buf] == pass + 1u) {
-            /* Rows that not every column sees hold inf or NaN, which a zero
-             * weight would turn into NaN. They are taken out of the tile,
-             * and the outputs of the columns that do see them become NaN
-             * at the end (as inf x weight parts gives in every kernel). */
-            for (uint32_t i = tid; i < PT * NB; i += NTHR) s_nan[i] = 0u;
-            __syncthreads();
-            for (uint32_t i = tid; i < PT * (HD / 8u); i += NTHR) {
-                const uint32_t p = i / (HD / 8u), pc = i % (HD / 8u), at = vaddr<VS>(p, pc);
-                uint32_t bits = 0u;
-                for (uint32_t e = 0; e < 8u; e++) {
-                    uint16_t *v = (uint16_t *)(s_v[buf][0] + at) + e;
-                    if ((*v & 0x7C00u) != 0x7C00u) continue;
-                    bits |= 1u << e;
-                    *v = 0u;
-                    if (G::NV == 2) ((uint16_t *)(s_v[buf][G::NV - 1u] + at))[e] = 0u;
-                }
-                if (bits) atomicOr(&s_nan[p * NB + pc / 4u], bits << (8u * (pc & 3u)));
-            }
-            __syncthreads();
-            for (uint32_t p = 0; p < PT && base + p < n_c; p++)
-                for (uint32_t b = 0; b < NB && sees(base + p); b++) {
-                    const uint32_t w = s_nan[p * NB + b] >> (4u * jg);
-                    nan_out |= ((uint64_t)(w & 15u) | (uint64_t)((w >> 16) & 15u) << 4) << (8u * b);
-                }
-        }
         /* ---- scores: tile tt holds positions base + 16 tt + 4 jg + i of
          * column c. Eight stages of two tiles and one block; the operands of
          * the stage after next are in flight, and the scales are applied one
@@ -544,6 +493,16 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
             for (uint32_t tt = 0; tt < NT; tt++) Sl[tt] = (f4_t){0.f, 0.f, 0.f, 0.f};
         }
         {
+            const uint8_t *kr = s_k[buf] + c * KS + 16u * jg;
+            const uint16_t *ksr = s_ks[KIND == Q4KV_Q8 ? buf : 0u] + 8u * jg;
+            h8_t A[8][2], ks[8];
+            auto fetch = [&](uint32_t st) {
+                const uint32_t b = st % NB, tp = st / NB;
+#pragma unroll
+                for (uint32_t k = 0; k < 2u; k++)
+                    A[st][k] = *(const h8_t *)(kr + (2u * tp + k) * 16u * KS + 64u * b);
+                if constexpr (KIND == Q4KV_Q8) ks[st] = *(const h8_t *)(ksr + st * 32u);
+            };
             f4_t C[8][2];
             auto scale = [&](uint32_t st) {
                 const uint32_t tp = st / NB;
@@ -553,6 +512,8 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
                     for (uint32_t i = 0; i < 4u; i++)
                         S[2u * tp + k][i] = fmaf((float)ks[st][4u * k + i], C[st][k][i], S[2u * tp + k][i]);
             };
+            fetch(0u);
+            fetch(1u);
 #pragma unroll
             for (uint32_t st = 0; st < 8u; st++) {
                 const uint32_t b = st % NB, tp = st / NB;
@@ -618,13 +579,74 @@ __global__ __launch_bounds__(512, 2) void qsa_dense_k(Args a) {
         mx *= qmul;
         /* this lane's positions only: the column's maximum is formed when a
          * lane passes the limit */
-        if (__ballot(mx > m_run + RESCALE_LOG2) != 0u) {
-            const float mn = max2(m_run, col_max(mx));
-            const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mn);
-            m_run = mn;
-            l_run *= alpha;
+        const uint32_t flag = __builtin_amdgcn_readfirstlane(flag_at);
+        const bool bad = masked && (flag & 0xFFFFu) == ((pass + 1u) & 0xFFFFu);
+        const bool grow = KIND == Q4KV_Q8 && !vq.big() && flag >> 16 == ((pass + 1u) & 0xFFFFu);
+        const bool up = __ballot(mx > m_run + RESCALE_LOG2) != 0u;
+        if (up || bad || grow) {
+            if (bad || grow) { /* the whole workgroup */
+                __syncthreads();
+                if (grow) {
+                    /* V over 128 from this pass on: its rows once more */
+                    vq.divide();
 #pragma unroll
-            for (uint32_t T = 0; T < TD; T++) acc[T] *= alpha;
+                    for (uint32_t T = 0; T < TD; T++) acc[T] *= VSCALE_STEP;
+#pragma unroll 1
+                    for (uint32_t i = tid; i < PT * (HD / 8u); i += NTHR) {
+                        const uint32_t p = i / (HD / 8u), pc = i % (HD / 8u), b = pc / 4u;
+                        const uint8_t *blk = vb + (size_t)min(base + p, n_all - 1u) * rstride + 34u * b;
+                        const h2_t vs = (h2_t)(__builtin_bit_cast(_Float16, ldg((const uint16_t *)blk)));
+                        u4_t wh, wl;
+#pragma unroll
+                        for (uint32_t e = 0; e < 4u; e++) {
+                            const uint32_t w = ldg((const uint16_t *)(blk + 2u + 8u * (pc & 3u)) + e) ^ 0x8080u;
+                            const h2_t f = vq.value(__builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)));
+                            const h2_t hi = f * vs;
+                            wh[e] = __builtin_bit_cast(uint32_t, hi);
+                            wl[e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(f, vs, -hi));
+                        }
+                        *(u4_t *)(s_v[buf][0] + vaddr<VS>(p, pc)) = wh;
+                        *(u4_t *)(s_v[buf][G::NV - 1u] + vaddr<VS>(p, pc)) = wl;
+                    }
+                    __syncthreads();
+                }
+                if (bad) {
+                    /* Rows that not every column sees hold inf or NaN, which a zero
+                     * weight would turn into NaN. They are taken out of the tile,
+                     * and the outputs of the columns that do see them become NaN
+                     * at the end (as inf x weight parts gives in every kernel). */
+                    for (uint32_t i = tid; i < PT * NB; i += NTHR) s_nan[i] = 0u;
+                    __syncthreads();
+                    for (uint32_t i = tid; i < PT * (HD / 8u); i += NTHR) {
+                        const uint32_t p = i / (HD / 8u), pc = i % (HD / 8u), at = vaddr<VS>(p, pc);
+                        uint32_t bits = 0u;
+                        for (uint32_t e = 0; e < 8u; e++) {
+                            uint16_t *v = (uint16_t *)(s_v[buf][0] + at) + e;
+                            if ((*v & 0x7C00u) != 0x7C00u) continue;
+                            bits |= 1u << e;
+                            *v = 0u;
+                            if (G::NV == 2) ((uint16_t *)(s_v[buf][G::NV - 1u] + at))[e] = 0u;
+                        }
+                        if (bits) atomicOr(&s_nan[p * NB + pc / 4u], bits << (8u * (pc & 3u)));
+                    }
+                    __syncthreads();
+                    for (uint32_t p = 0; p < PT && base + p < n_c; p++)
+                        for (uint32_t b = 0; b < NB && sees(base + p); b++) {
+                            const uint32_t w = s_nan[p * NB + b] >> (4u * jg);
+                            nan_out |= ((uint64_t)(w & 15u) | (uint64_t)((w >> 16) & 15u) << 4) << (8u * b);
+                        }
+                }
+                __syncthreads();
+                vfetch(0u);
+            }
+            if (up) {
+                const float mn = max2(m_run, col_max(mx));
+                const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - mn);
+                m_run = mn;
+                l_run *= alpha;
+#pragma unroll
+                for (uint32_t T = 0; T < TD; T++) acc[T] *= alpha;
+            }
         }
         const float ms = m_run == -INFINITY ? 0.f : m_run;
 #pragma unroll

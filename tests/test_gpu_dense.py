@@ -135,3 +135,29 @@ def test_scores_not_finite(rt, kind, hd):
         assert_attn_close(got[~hit], clean[~hit])
     for p in (kc, vc):
         rt.free(p)
+
+
+@pytest.mark.parametrize("hd", [256, 128])
+def test_inf_beside_a_large_scale(rt, hd):
+    """One pass holds a V row with an infinite scale and one with a scale past
+    512 (V goes over to v * scale / 128 there): tokens that do not see the
+    first are as without it, the others are not finite in its block only."""
+    n_head, n_kvh, n_tok, base = 16, 2, 300, 1500
+    note(f"dense inf beside a large scale hd={hd}")
+    ctx, bad, kh = base + n_tok, base + 170, 1
+    k, v, q, gate = _inputs(50 + hd, 2, n_head, n_kvh, hd, n_tok, ctx)
+    v[bad + 2, kh, :32] *= np.float32(1e6)
+    kc, _ = quantize_on_gpu(rt, k, 2)
+    vc, nb = quantize_on_gpu(rt, v, 2)
+    clean = _run(rt, q, gate, kc, vc, 2, n_kvh, base, ctx)
+    assert np.isfinite(clean).all() and np.abs(clean).max() > 1e3
+    rows = rt.download(vc, nb).reshape(ctx, n_kvh, -1).copy()
+    rows[bad, kh].view(np.uint16)[17] = 0x7C00
+    rt.h2d(vc, rows)
+    got = _run(rt, q, gate, kc, vc, 2, n_kvh, base, ctx)
+    hit = np.zeros(q.shape, bool)
+    hit[bad - base:, kh * n_head // n_kvh:, 32:64] = True
+    assert not np.isfinite(got[hit]).any()
+    assert np.array_equal(got[~hit], clean[~hit])
+    for p in (kc, vc):
+        rt.free(p)
