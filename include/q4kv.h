@@ -221,7 +221,8 @@ bool q4_hip_qsa_step_batch(const q4kv_step_desc *d_descs, uint32_t n_seq, uint32
  * allocates nothing. Same arguments, same split division and results as
  * q4_hip_qsa_step_batch, bit for bit. Returns false, with a message, when
  * the call's partials would exceed 4M floats (n_seq * n_kvh items x splits x
- * n_head/n_kvh x 258). Calls that overlap on one GPU share the array and
+ * n_head/n_kvh x 258; steps over q8_0 and f16 caches of 64 and 128 dims with up
+ * to 16 heads per KV head are cut to fit and never do). Calls that overlap on one GPU share the array and
  * race: order them on one stream. */
 bool q4_hip_qsa_step_batch_noalloc(const q4kv_step_desc *d_descs, uint32_t n_seq,
                                    uint32_t n_head, uint32_t n_kvh, uint32_t hd, float scale,

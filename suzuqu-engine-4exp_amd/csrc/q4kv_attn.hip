@@ -3320,7 +3320,8 @@ extern "C" bool q4_hip_qsa_decode_batch(const q4kv_seq_desc *d_descs, uint32_t n
 }
 
 /* The split plan q4_hip_qsa_step_batch's launch takes for these arguments
- * (the dispatch of step_batch below, then launch_kind's plan_launch). */
+ * (the dispatch of step_batch below, then launch_kind's plan_launch), where
+ * q4kv_rows_takes does not. */
 static Plan step_batch_plan(int kind, uint32_t hd, uint32_t n_items, uint32_t max_n,
                             uint32_t gqa, bool have, size_t cap) {
     if (any_shape(hd, gqa)) return Plan{false, 1u, any_splits(n_items, max_n, gqa, have, cap), 0u};
@@ -3415,8 +3416,13 @@ extern "C" bool q4_hip_qsa_step_batch_noalloc(const q4kv_step_desc *d_descs, uin
     /* the split division q4_hip_qsa_step_batch takes with the library's
      * buffer (so the same results) must fit the static scratch; planned on
      * the scratch's own capacity it is then the same division (every larger
-     * split count misses the larger buffer too) */
+     * split count misses the larger buffer too). The 64 / 128-dim kernel cuts
+     * its items to fit Q4KV_ROWS_PART in either buffer. */
+    static_assert(Q4KV_ROWS_PART <= Q4KV_SCRATCH_FLOATS, "partials of q4kv_rows_launch");
     const uint32_t gqa = n_head / n_kvh, n_items = n_seq * n_kvh;
+    if (q4kv_rows_takes(kv_f16, hd, gqa, true))
+        return step_batch(d_descs, n_seq, n_head, n_kvh, hd, scale, kv_f16, max_n,
+                          PartBuf{g_scratch_ptr[dev], Q4KV_SCRATCH_FLOATS});
     const Plan pl = step_batch_plan(kv_f16, hd, n_items, max_n, gqa, q4kv_part != nullptr,
                                     q4kv_part_cap);
     const uint32_t S = pl.S;

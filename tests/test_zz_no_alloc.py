@@ -105,3 +105,37 @@ def test_noalloc_rejects_partials_beyond_scratch(rt):
     assert not rt.lib.q4_hip_qsa_step_batch_noalloc(dummy, n_seq, N_KVH * gqa, N_KVH, 256,
                                                     1.0 / 16, q4kv.KV_Q8, 2051)
     rt.sync()
+
+
+@pytest.mark.parametrize("kind,hd", [(q4kv.KV_F16, 128), (q4kv.KV_Q8, 64)])
+def test_noalloc_takes_many_items_of_small_heads(rt, kind, hd):
+    """510 items of 16 heads per KV head at 64 / 128 dims: the plan of the
+    general kernels (2 splits, 4210560 floats) is not the one that runs; the
+    kernel of these shapes cuts its items to fit the scratch. Accepted, and the
+    same bits as q4_hip_qsa_step_batch."""
+    note(f"noalloc many items kind {kind} hd {hd}")
+    n_seq, n_head, ctx = 255, 32, 400
+    rng = np.random.default_rng(hd)
+    before = set(rt._owned)
+    cache = [rt.alloc(ctx * q4kv.token_bytes(kind, N_KVH, hd)) for _ in range(2)]
+    f32_to = rt.lib.q4_hip_f32_to_q8 if kind == q4kv.KV_Q8 else rt.lib.q4_hip_f32_to_f16
+    for c in cache:
+        assert f32_to(c, rt.upload(heads(rng, (ctx, N_KVH), hd=hd)), ctx * N_KVH * hd)
+    q = heads(rng, (n_seq, n_head), hd=hd)
+    dq, do = rt.upload(q), rt.alloc(q.nbytes)
+    kn, vn = (rt.upload(heads(rng, (N_KVH,), hd=hd)) for _ in range(2))
+    steps = (q4kv.StepDesc * n_seq)()
+    for i in range(n_seq):  # one cache; every item appends the same row to it
+        at = i * n_head * hd * 4
+        steps[i] = q4kv.StepDesc(q4kv.SeqDesc(*cache, dq + at, None, do + at, None, ctx, 0, ctx, 0),
+                                 kn, vn, ctx - 1)
+    dd = rt.upload(np.frombuffer(bytes(steps), np.uint8))
+    out = []
+    for entry in ("q4_hip_qsa_step_batch", "q4_hip_qsa_step_batch_noalloc"):
+        rt.h2d(do, np.full(q.size, np.nan, np.float32))
+        assert getattr(rt.lib, entry)(dd, n_seq, n_head, N_KVH, hd, 1.0 / np.sqrt(hd), kind, ctx), entry
+        rt.sync()
+        out.append(rt.download(do, q.nbytes, np.float32))
+    assert np.isfinite(out[0]).all() and np.array_equal(*out)
+    for p in [p for p in rt._owned if p not in before]:
+        rt.free(p)
