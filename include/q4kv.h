@@ -341,7 +341,7 @@ void q4_hip_host_free(void *p);
 bool q4kv_timer_begin(int slot);
 double q4kv_timer_end_ms(int slot);
 int q4kv_device_info(char *name, int name_len, int *n_cu, int *clock_khz);
-/* Arm per-launch event timing of the split-KV attention kernel for up to
+/* Arm per-launch event timing of the attention kernels (not their merges) for up to
  * max_launches launches; q4kv_prof_end waits and returns the number timed
  * and their summed duration in ms. */
 bool q4kv_prof_begin(int max_launches);

@@ -2547,8 +2547,13 @@ extern "C" int q4kv_prof_end(double *total_ms) {
     return g_prof_n;
 }
 
-static inline bool prof_armed(void) {
-    return g_prof_on && !q4kv_capturing && g_prof_n < g_prof_max;
+bool q4kv_prof_open(void) {
+    if (!g_prof_on || q4kv_capturing || g_prof_n >= g_prof_max) return false;
+    (void)hipEventRecord(g_pev[2 * g_prof_n], q4kv_stream);
+    return true;
+}
+void q4kv_prof_close(bool open) {
+    if (open) (void)hipEventRecord(g_pev[2 * g_prof_n++ + 1], q4kv_stream);
 }
 
 /* Workgroups a launch aims for (Q4KV_SPLIT_TARGET overrides, like the
@@ -3032,10 +3037,12 @@ static bool launch_sparse(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t
      * 1024 tokens, with and without it: 338 / 345 us at 2051 entries, 272 / 273
      * at 1536, 210 / 209 at 1024, 148 / 138 at 512 (a quarter of them window);
      * 512 tokens at 2051: 198 / 180. */
+    const bool prof = q4kv_prof_open();
     if (S == 1u && n_items >= 2048u && max_n > 1536u && band_enabled() && pb.ptr && q4kv_band_floats(n_items, gqa) <= pb.cap) {
         if (!q4kv_band_launch(a, n_items, pb.ptr)) return false;
     }
     if (!q4kv_sparse_launch(a, n_items)) return false;
+    q4kv_prof_close(prof);
     for (uint32_t i0 = 0; S > 1u && i0 < n_items; i0 += Q4KV_MAX_GRID_Y) {
         a.item0 = i0;
         const uint32_t ni = n_items - i0 < Q4KV_MAX_GRID_Y ? n_items - i0 : Q4KV_MAX_GRID_Y;
@@ -3136,8 +3143,7 @@ static bool launch_kind(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t g
             a.xgrp = ni / a.n_kvh * S;
             grid = dim3(8u * a.n_kvh * ((a.xgrp + 7u) / 8u), 1u, zg);
         }
-        const bool prof = prof_armed();
-        if (prof) (void)hipEventRecord(g_pev[2 * g_prof_n], q4kv_stream);
+        const bool prof = q4kv_prof_open();
         /* prefill through the slab kernel (one split): the shared recent
          * window of consecutive tokens goes to the band kernel first */
         a.band_nb = nullptr;
@@ -3196,7 +3202,7 @@ static bool launch_kind(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t g
             qsa_attn_k<KIND, IS_STEP(MODE) ? MODE_BATCH : MODE, 1><<<grid, 256, 0, q4kv_stream>>>(a);
         else
             qsa_attn_k<KIND, IS_STEP(MODE) ? MODE_BATCH : MODE, 2><<<grid, 256, 0, q4kv_stream>>>(a);
-        if (prof) (void)hipEventRecord(g_pev[2 * g_prof_n++ + 1], q4kv_stream);
+        q4kv_prof_close(prof);
         /* qsa_h16_k writes the q8_0 kernels' column order */
         if (S > 1u && !op && pl.h16)
             qsa_comb_k<Q4KV_Q8, MODE><<<dim3(gqa, ni), 256, 0, q4kv_stream>>>(a);

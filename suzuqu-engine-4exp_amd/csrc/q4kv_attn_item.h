@@ -208,6 +208,11 @@ __device__ static inline uint32_t split_pk(float x, float y, float nsel) {
     return pkrtz(__builtin_fmaf(nsel, h2lo(h), x), __builtin_fmaf(nsel, h2hi(h), y));
 }
 
+/* The timing of attention launches, while q4kv_prof_begin has armed it: events
+ * around the attention kernel (and the window's, not the merges). */
+bool q4kv_prof_open(void);
+void q4kv_prof_close(bool open);
+
 /* q8_0 V as the matrix products take it: v x scale in two fp16 parts, exact
  * for every scale below 512 (an int8 times an fp16: 19 bits, none below 2^-24;
  * 128 x 511.75 is still fp16). Whoever meets a larger finite scale goes over to

@@ -795,7 +795,9 @@ template <int HD> __global__ __launch_bounds__(256) void qsa_dense_merge_k(Args 
 
 template <int KIND, int HD> void launch(const Args &a) {
     const uint32_t grid = (a.T1 + (a.n_tiles - a.T1) * a.S) * a.n_kvh;
+    const bool prof = q4kv_prof_open();
     qsa_dense_k<KIND, HD><<<grid, NTHR, 0, q4kv_stream>>>(a);
+    q4kv_prof_close(prof);
     if (a.T1 < a.n_tiles) {
         const uint32_t cpw = 256u / (HD / 4u), c_hi = a.n_tok * a.gqa - a.T1 * COLS;
         qsa_dense_merge_k<HD><<<dim3((c_hi + cpw - 1u) / cpw, a.n_kvh), 256, 0, q4kv_stream>>>(a);

@@ -468,10 +468,12 @@ template <int KIND, int HD, int MODE> void launch(RowArgs ra, uint32_t n_items) 
     for (uint32_t i0 = 0; i0 < n_items; i0 += 65535u) {
         const uint32_t ni = std::min(n_items - i0, 65535u);
         ra.a.item0 = i0;
+        const bool prof = q4kv_prof_open();
         if (gqa <= 8u)
             qsa_rows_k<KIND, HD, MODE, 1><<<dim3(ra.S, ni), 256, 0, q4kv_stream>>>(ra);
         else
             qsa_rows_k<KIND, HD, MODE, 2><<<dim3(ra.S, ni), 256, 0, q4kv_stream>>>(ra);
+        q4kv_prof_close(prof);
         if (ra.S > 1u)
             qsa_rows_merge_k<HD, MODE><<<dim3(gqa, ni), 256, 0, q4kv_stream>>>(ra);
     }

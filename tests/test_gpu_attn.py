@@ -422,3 +422,33 @@ def test_config3_chunked_prefill_sampled(rt, oracle):
                        threads=8)
     assert_attn_close(got[ts], want, what="config3 sampled queries")
     assert np.all(np.isfinite(got))
+
+
+def test_launches_are_timed(rt):
+    """q4kv_prof_begin / q4kv_prof_end count one launch per attention call,
+    whichever kernel takes it: dense prefill, 64 / 128-dim decode, listed
+    prefill, 256-dim decode."""
+    note("timed launches")
+    rng = np.random.default_rng(77)
+    lib, before = rt.lib, set(rt._owned)
+    ctx, width, n_tok = 2000, 300, 300
+    bufs = {hd: [quantize_on_gpu(rt, heads(rng, (ctx, 2), hd=hd), 2)[0] for _ in range(2)]
+            for hd in (256, 128)}
+    q = rt.upload(heads(rng, (n_tok, 24)))
+    gate, out = rt.upload(np.zeros((n_tok, 24, 256), np.float32)), rt.alloc(n_tok * 24 * 1024)
+    sel = rt.upload(np.tile(np.arange(width, dtype=np.int32), (n_tok, 1)))
+    calls = [lambda: lib.q4_hip_qsa_decode_n(q, *bufs[256], gate, out, 24, 2, 256, n_tok,
+                                             ctx - n_tok, ctx, 1 / 16, 2),
+             lambda: lib.q4_hip_qsa_decode(q, *bufs[128], gate, out, 24, 2, 128, ctx, ctx, 0.09, 2),
+             lambda: lib.q4_hip_qsa_decode_idx(q, *bufs[256], gate, out, sel, width, 24, 2, 256,
+                                               n_tok, ctx, 1 / 16, 2),
+             lambda: lib.q4_hip_qsa_decode(q, *bufs[256], gate, out, 24, 2, 256, ctx, ctx, 1 / 16, 2)]
+    for k, call in enumerate(calls):
+        assert lib.q4kv_prof_begin(8)
+        for _ in range(3):
+            assert call()
+        ms = ctypes.c_double()
+        assert lib.q4kv_prof_end(ctypes.byref(ms)) == 3, k
+        assert 0.0 < ms.value < 100.0
+    for p in [p for p in rt._owned if p not in before]:
+        rt.free(p)
