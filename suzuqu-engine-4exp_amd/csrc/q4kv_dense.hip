@@ -934,7 +934,12 @@ bool q4kv_dense_launch(int kind, uint32_t hd, const float *q, const void *kc, co
     return q4kv_launch_ok("qsa dense prefill");
 }
 
-size_t q4kv_band_floats(uint32_t n_items, uint32_t gqa) { return (size_t)n_items * (1u + 2u * gqa); }
+/* n_items counts, then (m, l) pairs from an even offset (they are read and
+ * written as 8 bytes) */
+static size_t band_ml_at(uint32_t n_items) { return ((size_t)n_items + 1u) / 2u * 2u; }
+size_t q4kv_band_floats(uint32_t n_items, uint32_t gqa) {
+    return band_ml_at(n_items) + (size_t)n_items * 2u * gqa;
+}
 
 bool q4kv_band_launch(AttnArgs &a, uint32_t n_items, float *part) {
     const uint32_t gqa = a.n_head / a.n_kvh;
@@ -957,7 +962,7 @@ bool q4kv_band_launch(AttnArgs &a, uint32_t n_items, float *part) {
     b.kvh_stride = a.kvh_stride;
     b.width = a.width;
     b.band_nb = a.band_nb = (int32_t *)part;
-    b.band_ml = a.band_ml = part + n_items;
+    b.band_ml = a.band_ml = part + band_ml_at(n_items);
     qsa_dense_k<Q4KV_Q8, 256, true><<<b.n_tiles * a.n_kvh, NTHR, 0, q4kv_stream>>>(b);
     return q4kv_launch_ok("qsa band");
 }

@@ -43,6 +43,8 @@ def _lists(rng, n, width, ctx, run):
     (24, 2, 1026, 256, True, 256),   # lists that are all band
     (32, 2, 1030, 1537, False, 500), # the band apart, 16 heads
     (18, 2, 1025, 1600, True, 90),
+    (10, 1, 2049, 1539, False, 90),  # an odd number of items
+    (8, 1, 1601, 259, False, 70),    # the band and the slab kernel, odd
     (16, 2, 200, 259, False, 0),     # packed, 8 heads
     (4, 2, 220, 300, True, 64),      # packed, 2 heads
     (3, 3, 128, 290, False, 0),      # one head per KV head
