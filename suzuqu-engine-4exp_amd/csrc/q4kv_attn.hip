@@ -2964,7 +2964,8 @@ static Plan plan_launch(uint32_t hd, uint32_t n_items, uint32_t max_n, uint32_t 
     return pl;
 }
 
-/* The prefill band kernel (Q4KV_BAND=0 turns it off, for measurement). */
+/* The shared window of listed prefill apart (qsa_dense_k with BAND;
+ * Q4KV_BAND=0 leaves it in the lists, for measurement). */
 static bool band_enabled(void) {
     static int v = -1;
     if (v < 0) {
@@ -3113,7 +3114,7 @@ static bool launch_kind(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t g
     bool app = false;
     if constexpr (KIND == Q4KV_Q8 && (MODE == MODE_INDEXED || MODE == MODE_DENSE)) {
         /* the chunk kernel's single-buffer instance, or the slab kernel on
-         * decode-sized launches (prefill-sized ones run the band kernel
+         * decode-sized launches (prefill-sized ones run the window's tiles
          * first, which reads the rows without the substitution) */
         app = a.hd == 256u && n_items <= 64u && held_matches(a) &&
               ((chunk && !pl.slab && cps < db_min_chunks()) ||
@@ -3145,7 +3146,8 @@ static bool launch_kind(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t g
         }
         const bool prof = q4kv_prof_open();
         /* prefill through the slab kernel (one split): the shared recent
-         * window of consecutive tokens goes to the band kernel first */
+         * window of consecutive tokens goes to the dense kernel's tiles
+         * first */
         a.band_nb = nullptr;
         a.band_ml = nullptr;
         if (MODE == MODE_INDEXED && KIND == Q4KV_Q8 && pl.slab && S == 1u && gqa <= 8u &&

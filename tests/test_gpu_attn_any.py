@@ -253,7 +253,7 @@ def test_wide_prefill_multi_pass(rt, oracle, kind, n_head):
 def test_unaligned_caches(rt, oracle, kind, n_head, n_tok, off):
     """Caches that are not 16-byte aligned (base + off bytes) take kernels that
     read them in smaller pieces; results as for aligned caches. The 600-token
-    q8_0 case is prefill-sized (otherwise the band and slab kernels)."""
+    q8_0 case is prefill-sized (otherwise the listed prefill kernel)."""
     note(f"unaligned caches kind={kind} n_head={n_head} n_tok={n_tok} off={off}")
     rng = np.random.default_rng(1400 + kind + n_head + n_tok)
     n_kvh, hd, ctx, width = 2, 256, 5000, 2051

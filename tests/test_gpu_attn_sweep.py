@@ -1,8 +1,8 @@
 """Seeded randomized parity sweep of the attention entry points against the
 oracle (|got - ref| <= 2e-3 + 1e-3*|ref|): cache width, head_dim, query heads
 per KV head, KV heads, token count, entry point and list shape are drawn per
-case, so the kernel choice (chunk, slab, band, f16, f32, general-shape and
-generic kernels, one or many splits) varies across cases. Each case is
+case, so the kernel choice (chunk, slab, listed and dense prefill, 64 /
+128-dim, f16, f32, general-shape and generic kernels, one or many splits) varies across cases. Each case is
 small enough for the oracle; the case parameters are printed before its GPU
 step. List shapes follow the reference's format (src/q4_rocm.cu:7668-7696):
 positions, -1 padding, and here also out-of-range entries, duplicates,

@@ -12,7 +12,8 @@ oracle (|got - ref| <= 2e-3 + 1e-3*|ref|):
   more than 1024 positions falls back to the general kernel);
 - runs longer than 1024 positions (the band takes their last 1024);
 - right-aligned lists (-1 padding first, then a run from position 0);
-- a token count that is not a multiple of the 16-token band tile;
+- a token count that is not a multiple of the band tile (16 tokens at 8 heads
+  per KV head, 32 at fewer);
 - 8, 4 and 1 query heads per KV head, with and without the gate.
 
 src/q4_rocm.cu:6816-6861 is the list semantics (padding and out-of-range
@@ -26,7 +27,7 @@ from test_gpu_attn import gpu_idx_kv
 
 pytestmark = pytest.mark.gpu
 
-N_TOK = 4200  # 8400 items with two KV heads: one split each; 4200 % 16 == 8
+N_TOK = 4200  # 8400 items with two KV heads: one split each; 4200 % 16 == 4200 % 32 == 8
 
 
 def _prefix(rng, lo, hi, count):

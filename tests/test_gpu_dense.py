@@ -37,20 +37,37 @@ def _inputs(seed, kind, n_head, n_kvh, hd, n_tok, ctx):
     return k, v, q, rng.standard_normal(q.shape).astype(np.float32)
 
 
+def _reaches_dense(hd, n_tok, n_head, n_kvh, kind, max_n):
+    """q4kv_dense_takes for aligned caches: other calls run q4kv_rows.hip or
+    the 256-dim decode kernels."""
+    gqa = n_head // n_kvh
+    if gqa > 16:
+        return True
+    hg = 2 if gqa > 8 else 1
+    slots = n_tok * n_kvh * hg * (max_n - min(max_n, n_tok) // 2)
+    tiles = -(-n_tok * gqa // 128) * n_kvh
+    per_tile = n_tok * n_kvh * hg / tiles * min(1.0, tiles * 64 / 256)
+    return (n_tok > 1 and slots > (280000 if hd == 256 else 160000)
+            and per_tile > (1.5 if kind == q4kv.KV_F16 or hd == 64 else 2 if hd == 128 else 4))
+
+
 # (kind, n_head, n_kvh, hd, n_tok, base, max_kv below base + n_tok, shift)
 CASES = [
-    (2, 24, 2, 256, 301, 640, 0, 0),    # 28.2 tiles, unsplit and split
+    (2, 24, 2, 256, 301, 640, 0, 0),    # 28.2 tiles in 4 splits
     (2, 24, 2, 256, 700, 0, 0, 0),      # causal from position 0: the last tiles split
     (1, 16, 2, 256, 130, 1999, 0, 0),   # f16
     (2, 8, 2, 256, 600, 700, 0, 1),     # 4 heads per KV head, unaligned queries
     (2, 20, 1, 256, 9, 33, 0, 0),       # more than 16 heads per KV head
     (2, 16, 2, 256, 280, 1000, 150, 0), # the cache ends before the tokens do
-    (1, 32, 8, 128, 33, 95, 0, 0),      # 128 dims, 64 positions per pass
-    (2, 32, 8, 128, 1, 5000, 0, 0),     # one token, many splits
-    (2, 3, 1, 128, 65, 62, 40, 3),      # KV rows of 136 bytes
-    (1, 24, 8, 64, 43, 127, 0, 0),      # 64 dims, 128 positions per pass
-    (2, 16, 4, 64, 2, 0, 0, 0),         # the smallest prompt
-    (2, 4, 4, 64, 129, 3000, 0, 0),     # one head per KV head
+    (1, 32, 8, 128, 133, 195, 0, 0),    # 128 dims, 64 positions per pass
+    (1, 16, 2, 128, 201, 3001, 0, 1),   # its tiles in 8 splits, unaligned queries
+    (2, 32, 8, 128, 47, 2003, 0, 0),    # 12 splits, a tile of 60 columns
+    (2, 40, 2, 128, 1, 5000, 0, 0),     # one token, 32 splits
+    (2, 3, 1, 128, 705, 62, 40, 3),     # KV rows of 136 bytes, 6 splits
+    (1, 24, 8, 64, 143, 127, 0, 0),     # 64 dims, 128 positions per pass
+    (1, 24, 2, 64, 83, 2900, 0, 0),     # 12 splits
+    (2, 36, 2, 64, 2, 0, 0, 0),         # the smallest prompt
+    (2, 4, 4, 64, 129, 3000, 0, 0),     # one head per KV head, 12 splits
 ]
 
 
@@ -58,6 +75,7 @@ CASES = [
 def test_dense_prefill(rt, oracle, kind, n_head, n_kvh, hd, n_tok, base, cut, shift):
     note(f"dense kind={kind} heads={n_head}/{n_kvh} hd={hd} n_tok={n_tok} base={base} cut={cut}")
     ctx = base + n_tok
+    assert _reaches_dense(hd, n_tok, n_head, n_kvh, kind, ctx - cut)
     k, v, q, gate = _inputs(31 * hd + n_tok, kind, n_head, n_kvh, hd, n_tok, ctx)
     kc, _ = quantize_on_gpu(rt, k, kind)
     vc, _ = quantize_on_gpu(rt, v, kind)

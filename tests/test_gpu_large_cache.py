@@ -5,8 +5,8 @@ of 4.3M; f32: 2048 bytes, from 2.1M of 2.2M). Only the rows the lists name
 are written; the oracle runs on a compact copy of those rows with the
 lists renumbered, so the host holds no multi-GiB arrays. Paths: one-token
 decode (chunk, slab, f16, f32 and general-shape kernels), the fused step
-and q4_hip_kv_append_d appending at the cache's last position, and a
-prefill-sized launch (band + slab kernels). A
+and q4_hip_kv_append_d appending at the cache's last position, and
+prefill launches (the listed kernel; the shared window + slab kernel). A
 byte offset computed in 32 bits would read or write the wrong rows here."""
 import ctypes
 
@@ -92,7 +92,8 @@ def _setup(rt, oracle, rng, kind, n_tok, pool_n):
     (q4kv.KV_F16, 16, 1),   # f16 kernel
     (q4kv.KV_F32, 16, 1),   # f32 kernel
     (q4kv.KV_Q8, 40, 1),    # general-shape kernel (20 query heads per KV head)
-    (q4kv.KV_Q8, 16, 600),  # prefill-sized: band + slab kernels
+    (q4kv.KV_Q8, 16, 600),  # the listed prefill kernel
+    (q4kv.KV_Q8, 16, 800),  # the shared window's tiles + the slab kernel
 ])
 def test_decode_past_4gib(rt, oracle, kind, n_head, n_tok):
     note(f"large cache decode kind={kind} n_head={n_head} n_tok={n_tok}")

@@ -6,7 +6,7 @@ the softmax scale where a kernel folds it in) by the power of two that
 brings its largest magnitude into [0.5, 1), so no range of q is excluded
 and the results must not depend on the magnitude:
 test_query_magnitude_any runs queries x 1e5 and x 1e-4 through every MFMA
-kernel (chunk, slab, band, f16, f32, generic). Here one 32-dimension
+kernel (chunk, slab, listed prefill, window, f16, f32, 128 dims). Here one 32-dimension
 block of every head sums to about +704 and another to about -640 (about +63
 and -58 after the scale): a kernel that folded the +1152 bias of its
 int8 -> fp16 K operands into a product with those sums (-1152 x 63 is
@@ -24,9 +24,9 @@ pytestmark = pytest.mark.gpu
 
 
 # (query heads, tokens): decode through the chunk kernel (8 per KV head) and
-# the slab kernel (16); prefill-sized launches through the band + slab
-# kernels (8 and 16 per KV head)
-@pytest.mark.parametrize("n_head,n_tok", [(16, 1), (32, 1), (16, 700), (32, 300)])
+# the slab kernel (16); prefill through the listed kernel (8 and 16 per KV
+# head) and, from 1536 items on, the shared window's tiles and the slab kernel
+@pytest.mark.parametrize("n_head,n_tok", [(16, 1), (32, 1), (16, 700), (32, 300), (16, 800)])
 def test_large_query_blocks(rt, oracle, n_head, n_tok):
     n_kvh, hd, width = 2, 256, 2051
     note(f"large query blocks n_head={n_head} n_tok={n_tok}")
@@ -62,10 +62,10 @@ def test_large_query_blocks(rt, oracle, n_head, n_tok):
                       combined=True)
 
 
-@pytest.mark.parametrize("n_head,n_tok", [(16, 1), (32, 1), (16, 700), (32, 300)])
+@pytest.mark.parametrize("n_head,n_tok", [(16, 1), (32, 1), (16, 700), (32, 300), (16, 800)])
 def test_large_v_values(rt, oracle, n_head, n_tok):
-    """V values up to ~2.4e4 (block scales up to ~190; the band kernel's fp16
-    parts of v * scale stay below 65504), K and Q at unit scale. The outputs
+    """V values up to ~2.4e4 (block scales up to ~190, v * scale still
+    inside fp16), K and Q at unit scale. The outputs
     are the unit-scale outputs times 1000, so the bar is the unit-scale bar
     times 1000: |got - ref| <= 2 + 1e-3*|ref|. (The chunk and slab kernels
     carry V as 1152 + v and remove the bias on the MFMA pipe, so their error
@@ -99,10 +99,11 @@ def test_large_v_values(rt, oracle, n_head, n_tok):
 
 
 # (kind, head_dim, query heads, tokens): the chunk kernel (q8, 8 per KV
-# head), the slab kernel (16), the band + slab prefill kernels, the f16
-# kernel (8 and 16), the f32 kernel, the generic MFMA kernel (q8, hd 128)
+# head), the slab kernel (16), listed prefill, the shared window + slab
+# kernel, the f16 kernel (8 and 16), the f32 kernel, the 128-dim kernel
 @pytest.mark.parametrize("kind,hd,n_head,n_tok", [(2, 256, 16, 1), (2, 256, 32, 1),
-                                                  (2, 256, 16, 300), (1, 256, 16, 1),
+                                                  (2, 256, 16, 300), (2, 256, 16, 800),
+                                                  (1, 256, 16, 1),
                                                   (1, 256, 32, 1), (0, 256, 16, 1),
                                                   (2, 128, 16, 1)])
 @pytest.mark.parametrize("qscale", [1e5, 1e-4])
