@@ -119,3 +119,39 @@ def test_prefill_band_split(rt, oracle, n_head, width, gated, long_run):
             if not (sel[t, kh] >= 0).any():
                 g = n_head // n_kvh
                 assert not got[t, kh * g:(kh + 1) * g].any(), (t, kh)
+
+
+@pytest.mark.parametrize("n_head,width", [
+    (8, 40), (8, 64), (6, 70), (16, 63), (16, 150), (10, 200), (2, 129),
+])
+def test_narrow_lists(rt, oracle, n_head, width):
+    """Lists of a few dozen entries, down to less than a window: every token of
+    a tile (16 to 32, in one to four rounds of the waves), runs of 63 and 64,
+    whole-list runs, padding on either side, a ragged last tile."""
+    n_kvh, hd, n_tok = 2, 256, 1037
+    note(f"narrow lists n_head={n_head} width={width}")
+    rng = np.random.default_rng(n_head * 1000 + width)
+    base, ctx = 500, 500 + n_tok
+    k, v = heads(rng, (ctx, n_kvh)), heads(rng, (ctx, n_kvh))
+    q = heads(rng, (n_tok, n_head))
+    kc, _ = quantize_on_gpu(rt, k, 2)
+    vc, _ = quantize_on_gpu(rt, v, 2)
+    sel = np.full((n_tok, n_kvh, width), -1, np.int32)
+    for t in range(n_tok):
+        for kh in range(n_kvh):
+            cat, end = (t + kh) % 6, base + t
+            n = width if cat < 4 else width - width // 3
+            rr = min(n, (63, 64, n, 5)[cat % 4])
+            row = np.concatenate([_prefix(rng, 0, end - rr, n - rr), np.arange(end - rr + 1, end + 1)])
+            at = width - n if cat == 4 else 0  # padding first, or last
+            sel[t, kh, at:at + n] = row
+    sel[n_tok // 2] = -1
+    got = gpu_idx_kv(rt, q, kc, vc, 2, n_head, n_kvh, hd, sel.ravel(), width,
+                     n_kvh * width, width, ctx)
+    rt.free(kc)
+    rt.free(vc)
+    want = oracle.attn(q, oracle.quant_q8(k), oracle.quant_q8(v), 2, n_head, n_kvh, hd, n_tok,
+                       idx=sel.ravel(), width=width, tok_stride=n_kvh * width, kvh_stride=width,
+                       max_kv=ctx, threads=8)
+    assert_attn_close(got, want, what=f"narrow lists n_head={n_head} width={width}")
+    assert not got[n_tok // 2].any()
