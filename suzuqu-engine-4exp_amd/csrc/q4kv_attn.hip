@@ -3022,13 +3022,45 @@ static bool sparse_takes(uint32_t n_items, uint32_t max_n, uint32_t gqa) {
     return gqa > 8u ? n_items > 16u && (uint64_t)n_items * max_n >= 60000u
                     : n_items >= 384u && n_items < 1536u;
 }
+/* Splits of a listed prefill launch, and whether the KV heads of a token that
+ * share its list (their rows are adjacent) go to one XCD (xgrp: the tokens, or
+ * 0; the grid is then padded to whole rows of eight tokens). A CU holds two
+ * workgroups, which share its pipes, and they are handed out in turn, padding
+ * included: a launch of a few more than one each takes nearly as long as one of
+ * two each. 5 + p passes of a wave against 6.7 + 1.45 p, in units of 3.1 us
+ * (24 / 2 and 16 / 1 heads, 16 to 200 tokens, 600 to 2051 entries). 2051
+ * entries, 24 / 2 heads, 17 tokens: 8 grouped splits (384 workgroups, 272 of
+ * them real) 30 us, the chunk kernel 25; 24 tokens: 8 splits 30.5, 5 splits
+ * 26.9; 16 / 1 heads, 40 tokens: 8 splits 32.3, 6 splits 25.1, the chunk
+ * kernel 26.9; 192 items: 2 splits 61.7, one 67.9. */
+static uint32_t sparse_split(const AttnArgs &a, uint32_t n_items, uint32_t max_n, uint32_t gqa,
+                             const PartBuf &pb, uint32_t &xgrp) {
+    const uint32_t n_pass = (max_n + 31u) / 32u, tok = n_items / a.n_kvh;
+    const bool shared = a.kvh_stride == 0u && a.n_kvh > 1u && n_items % a.n_kvh == 0u;
+    uint32_t top = n_items < 512u ? 512u / n_items : 1u, best = 1u; /* the resident workgroups once */
+    if (top > n_pass / 8u) top = n_pass / 8u;
+    if (top < 1u || !pb.ptr) top = 1u;
+    xgrp = shared ? tok : 0u;
+    uint32_t least = ~0u;
+    for (uint32_t S = top; S >= 1u && top > 1u; S--) {
+        if (S > 1u && (size_t)n_items * S * gqa * PSTRIDE > pb.cap) continue;
+        const uint32_t p = ((n_pass + S - 1u) / S + 3u) / 4u;
+        for (uint32_t group = shared ? 2u : 1u; group-- > 0u;) {
+            /* workgroups per XCD of 32 CUs */
+            const uint32_t wgs = group ? (tok + 7u) / 8u * a.n_kvh * S : (n_items * S + 7u) / 8u;
+            const uint32_t cost = wgs <= 32u ? 500u + 100u * p : 670u + 145u * p;
+            if (cost < least) {
+                least = cost;
+                best = S;
+                xgrp = group ? tok : 0u;
+            }
+        }
+    }
+    return best;
+}
 static bool launch_sparse(AttnArgs a, uint32_t n_items, uint32_t max_n, uint32_t gqa, PartBuf pb) {
     if (!a.kc || !a.vc || !a.q || !a.out || !q4kv_flush()) return false;
-    const uint32_t n_pass = (max_n + 31u) / 32u;
-    uint32_t S = n_items < 512u ? 512u / n_items : 1u; /* the resident workgroups once */
-    if (S > n_pass / 8u) S = n_pass / 8u;
-    if (S < 1u || !pb.ptr) S = 1u;
-    while (S > 1u && (size_t)n_items * S * gqa * PSTRIDE > pb.cap) S--;
+    const uint32_t S = sparse_split(a, n_items, max_n, gqa, pb, a.xgrp);
     a.S = S;
     a.part = pb.ptr;
     a.item0 = 0u;

@@ -250,7 +250,8 @@ bool q4kv_rows_launch(int kind, int mode, const AttnArgs &a, uint32_t n_items, u
 
 /* Listed attention of many items over a q8_0 cache, hd 256, up to 16 query
  * heads per KV head (q4kv_sparse.hip): a.S splits of each list, partials in
- * natural column order. */
+ * natural column order; a.xgrp: the tokens, where a token's KV heads share its
+ * list and go to one XCD, or 0. */
 bool q4kv_sparse_launch(const AttnArgs &a, uint32_t n_items);
 
 /* The shared recent window of consecutive prefill tokens' lists (q8_0, hd

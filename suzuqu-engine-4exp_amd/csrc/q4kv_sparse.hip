@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t c = lane & 15u, jg = lane >> 4, kk = c & 3u;
     uint32_t s, item;
-    /* KV heads that share a list on one XCD (their rows are adjacent) */
+    /* KV heads that share a list on one XCD (their rows are adjacent; xgrp) */
     {
         s = blockIdx.x % a.S;
         const uint32_t L = blockIdx.x / a.S;
@@ -477,15 +477,9 @@ __global__ __launch_bounds__(256, 2) void qsa_sparse_k(AttnArgs a) {
 
 } // namespace
 
-bool q4kv_sparse_launch(const AttnArgs &a0, uint32_t n_items) {
-    AttnArgs a = a0;
+bool q4kv_sparse_launch(const AttnArgs &a, uint32_t n_items) {
     const uint32_t gqa = a.n_head / a.n_kvh;
-    uint32_t slots = n_items;
-    a.xgrp = 0u;
-    if (a.kvh_stride == 0u && a.n_kvh > 1u && n_items % a.n_kvh == 0u) {
-        a.xgrp = n_items / a.n_kvh;
-        slots = (a.xgrp + 7u) / 8u * 8u * a.n_kvh;
-    }
+    const uint32_t slots = a.xgrp ? (a.xgrp + 7u) / 8u * 8u * a.n_kvh : n_items;
     if (gqa <= 8u)
         qsa_sparse_k<true><<<slots * a.S, 256, 0, q4kv_stream>>>(a);
     else

@@ -37,6 +37,9 @@ def _lists(rng, n, width, ctx, run):
 # band; 9 to 16 and 1 to 8 heads per KV head
 @pytest.mark.parametrize("n_head,n_kvh,n_tok,width,per_kvh,run", [
     (24, 2, 16, 2051, False, 0),     # 8 splits of 8 passes or more
+    (24, 2, 17, 2051, False, 0),     # 7 splits, a token's KV heads not on one XCD
+    (24, 2, 24, 2051, False, 90),    # 5 splits, grouped again
+    (16, 1, 41, 2051, False, 0),     # 6 splits
     (24, 2, 130, 300, False, 70),    # one split
     (18, 2, 140, 257, True, 0),
     (32, 2, 1030, 261, False, 90),   # many tokens, short lists: the band stays in them
